@@ -16,9 +16,9 @@ OBJDIR = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libhymd_amd.so")
 ARCH = os.environ.get("HYMD_OFFLOAD_ARCH", "gfx950")
 
-SOURCES = ["common.hip", "scan.hip", "fft.hip", "field.hip", "batch.hip", "bonded.hip", "integrator.hip", "fused.hip",
+SOURCES = ["common.hip", "scan.hip", "fft.hip", "xline.hip", "xline_fixed.hip", "xline_34.hip", "xline_56.hip", "xline_78.hip", "field.hip", "batch.hip", "bonded.hip", "integrator.hip", "fused.hip",
            "md.hip", "thermostat.hip", "topology.hip"]
-HEADERS = ["common.h", "fft.h", "field_dev.h", "bonded.h"]
+HEADERS = ["common.h", "fft.h", "fft_line.h", "fft_ct.h", "xline.h", "field_dev.h", "bonded.h"]
 
 
 def _hipcc():

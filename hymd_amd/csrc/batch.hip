@@ -29,7 +29,7 @@ struct RepGeom {
     int64_t grid_off;  // float offset of its T real grids
     int64_t spec_off;  // complex offset of its T spectra
     int64_t part_off;  // first partial row
-    int64_t grad_off;  // complex offset of its 3T gradient spectra
+    int64_t grad_off;  // complex offset of its 2T x-inverse spectra
     int64_t fgrid_off; // float offset of its 3T force grids
     double inv_h[3];
     double kfac[3];
@@ -158,15 +158,14 @@ __global__ void __launch_bounds__(kBlock) batch_paint_rows_kernel(const float4 *
     }
 }
 
-// grid (k-space blocks, slots of the group): the gradient spectra
-// -i k_d V_t of each replica, V_t = H sum_s A_ts H rho_s / G, with the
-// arithmetic of the single-mesh k-space pass (field.hip), so each replica's
-// force grids equal hymd_field_moments' bit for bit.  coupling: per slot T x T.
+// grid (k-space blocks, slots of the group): -i k_x V_t and V_t of each
+// replica (no shift: V_t = H sum_s A_ts H rho_s / G), by the single-mesh pass's
+// kspace_point, so each replica's force grids equal hymd_field_moments' bit for
+// bit.  par: per slot, built by the host.
 template <int MAXT>
 __global__ void __launch_bounds__(kBlock) batch_kspace_kernel(const float2 *__restrict__ spec,
-                                                               const RepGeom *__restrict__ geo, int slot0, int T,
-                                                               const double *__restrict__ sigma2,
-                                                               const double *__restrict__ coupling,
+                                                               const RepGeom *__restrict__ geo, int slot0,
+                                                               const FieldK *__restrict__ par,
                                                                float2 *__restrict__ grad) {
     const int slot = slot0 + (int)blockIdx.y;
     const RepGeom &G = geo[slot];
@@ -177,39 +176,10 @@ __global__ void __launch_bounds__(kBlock) batch_kspace_kernel(const float2 *__re
     g.zh = G.zh;
     g.gc = G.gc;
     for (int d = 0; d < 3; ++d) g.kfac[d] = G.kfac[d];
-    const double s2 = sigma2[slot], inv_g = 1.0 / (double)G.g;
-    const double *A = coupling + (int64_t)slot * T * T;
-    const float2 *sp = spec + G.spec_off;
-    float2 *gr = grad + G.grad_off;
+    const FieldK &p = par[slot];
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t kk = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; kk < g.gc; kk += stride) {
-        double k[3], kd[3], wgt;
-        kvec(g, kk, k, kd, wgt);
-        const double k2 = k[0] * k[0] + k[1] * k[1] + k[2] * k[2];
-        const float H = (float)exp(-0.5 * s2 * k2);
-        const float hn = (float)((double)H * inv_g);
-        float2 ph[MAXT];
-#pragma unroll
-        for (int t = 0; t < MAXT; ++t)
-            if (t < T) ph[t] = cscale(sp[(int64_t)t * g.gc + kk], hn);
-#pragma unroll
-        for (int t = 0; t < MAXT; ++t) {
-            if (t >= T) continue;
-            float2 v = make_float2(0.f, 0.f);
-#pragma unroll
-            for (int u = 0; u < MAXT; ++u)
-                if (u < T) {
-                    const float a = (float)A[t * T + u];
-                    v.x += a * ph[u].x;
-                    v.y += a * ph[u].y;
-                }
-            v = cscale(v, H);
-            float2 *gt = gr + (int64_t)(3 * t) * g.gc + kk;
-            gt[0] = make_float2((float)kd[0] * v.y, -(float)kd[0] * v.x);
-            gt[g.gc] = make_float2((float)kd[1] * v.y, -(float)kd[1] * v.x);
-            gt[2 * g.gc] = make_float2((float)kd[2] * v.y, -(float)kd[2] * v.x);
-        }
-    }
+    for (int64_t kk = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; kk < g.gc; kk += stride)
+        kspace_point<MAXT>(spec + G.spec_off, grad + G.grad_off, nullptr, g, p, kk);
 }
 
 // Forces of the binned particles: each reads its replica's 3 force grids of
@@ -308,8 +278,9 @@ struct hymd_batch {
     DevBuf d_chunk_in, d_chunk_binned, d_pstart, d_row_slot;  // lookup tables (see the kernels)
     DevBuf keys, perm, xs, counts, start, tiles;  // xs: binned records (x, y, z, type bits)
     DevBuf rho, spec, partials, result;
-    DevBuf grad, fgrid, d_coupling;  // force stages: 3T spectra and grids per replica, T x T coupling per slot
-    HostBuf h_sigma2, h_result, h_coupling;
+    DevBuf grad, fgrid, d_par;  // force stages: 2T spectra and 3T grids per replica, k-space parameters per slot
+    DevBuf d_kf, tmp;           // per slot k_y and k_z factors; the line passes' scratch
+    HostBuf h_sigma2, h_result, h_par;
     int64_t grad_total = 0, fgrid_total = 0;
     int max_mz = 0;
     // captured sequences: [0] moments, [1] moments + forces
@@ -327,6 +298,18 @@ struct hymd_batch {
         if (stream) (void)hipStreamDestroy(stream);
     }
 };
+
+// The force grids of a group from its x-inverse spectra.
+static YzJob force_job(const hymd_batch *b, const RepGroup &gp) {
+    const RepGeom &G0 = b->geo[gp.first];
+    YzJob job;
+    job.T = b->T;
+    job.systems = gp.count;
+    job.kf = (const double2 *)b->d_kf.ptr + gp.first;
+    job.in = (const float2 *)b->grad.ptr + G0.grad_off;
+    job.force = (float *)b->fgrid.ptr + G0.fgrid_off;
+    return job;
+}
 
 // forces (device (n,3)) or NULL: the moments only
 static int batch_enqueue(hymd_batch *b, const float *x, const int32_t *types, float *forces) {
@@ -372,19 +355,18 @@ static int batch_enqueue(hymd_batch *b, const float *x, const int32_t *types, fl
         HYMD_HIP(hipGetLastError());
         if (forces) {
             dim3 kgrid((unsigned)std::min(grid_for(G0.gc), 1024), (unsigned)gp->count);
-            const double *cp = (const double *)b->d_coupling.ptr;
+            const FieldK *par = (const FieldK *)b->d_par.ptr;
             float2 *grad = (float2 *)b->grad.ptr;
             if (b->T <= 4)
                 batch_kspace_kernel<4><<<kgrid, kBlock, 0, s>>>((const float2 *)b->spec.ptr,
-                                                                (const RepGeom *)b->d_geo.ptr, gp->first, b->T,
-                                                                (const double *)b->d_sigma2.ptr, cp, grad);
+                                                                (const RepGeom *)b->d_geo.ptr, gp->first, par, grad);
             else
                 batch_kspace_kernel<8><<<kgrid, kBlock, 0, s>>>((const float2 *)b->spec.ptr,
-                                                                (const RepGeom *)b->d_geo.ptr, gp->first, b->T,
-                                                                (const double *)b->d_sigma2.ptr, cp, grad);
+                                                                (const RepGeom *)b->d_geo.ptr, gp->first, par, grad);
             HYMD_HIP(hipGetLastError());
-            HYMD_TRY(fft_c2r(gp->plan, grad + G0.grad_off, (float *)b->fgrid.ptr + G0.fgrid_off,
-                             gp->count * 3 * b->T, 1.f, s));
+            HYMD_TRY(fft_inverse_x(gp->plan, grad + G0.grad_off, gp->count * 2 * b->T, s));
+            const YzJob job = force_job(b, *gp);
+            HYMD_TRY(fft_yz_multi(gp->plan, job, (float2 *)b->tmp.ptr, s));
         }
     }
     if (forces && b->n > 0) {
@@ -473,7 +455,7 @@ extern "C" int hymd_batch_create(hymd_batch **out, int32_t n_replicas, const int
             G.spec_off = soff;
             G.nb = moments_blocks(G.gc);
             G.part_off = poff;
-            G.grad_off = 3 * soff;
+            G.grad_off = 2 * soff;
             G.fgrid_off = 3 * goff;
             rows += G.mx * G.my;
             goff += (int64_t)T * G.g;
@@ -498,7 +480,7 @@ extern "C" int hymd_batch_create(hymd_batch **out, int32_t n_replicas, const int
     for (const RepGeom &G : b->geo) b->max_mz = std::max(b->max_mz, G.mz);
     HYMD_REQUIRE((int64_t)T * b->max_mz <= 2048, "n_types x the largest z edge must be <= 2048 (got %d x %d)", T,
                  b->max_mz);
-    b->grad_total = 3 * soff;
+    b->grad_total = 2 * soff;
     b->fgrid_total = 3 * goff;
     const size_t nn = (size_t)std::max<int64_t>(b->n, 1);
     std::vector<int> nbs(R);
@@ -548,8 +530,11 @@ extern "C" int hymd_batch_create(hymd_batch **out, int32_t n_replicas, const int
     HYMD_TRY(b->result.reserve(sizeof(double) * b->row_len * R));
     HYMD_TRY(b->h_sigma2.reserve(sizeof(double) * R));
     HYMD_TRY(b->h_result.reserve(sizeof(double) * b->row_len * R));
-    HYMD_TRY(b->h_coupling.reserve(sizeof(double) * T * T * R));
-    HYMD_TRY(b->d_coupling.reserve(sizeof(double) * T * T * R));
+    HYMD_TRY(b->h_par.reserve(sizeof(FieldK) * R));
+    HYMD_TRY(b->d_par.reserve(sizeof(FieldK) * R));
+    HYMD_TRY(b->d_kf.reserve(sizeof(double2) * R));
+    std::vector<double2> kf(R);
+    for (int sl = 0; sl < R; ++sl) kf[sl] = make_double2(b->geo[sl].kfac[1], b->geo[sl].kfac[2]);
     hipStream_t s = b->stream;
     HYMD_HIP(hipMemcpyAsync(b->d_geo.ptr, b->geo.data(), sizeof(RepGeom) * R, hipMemcpyHostToDevice, s));
     HYMD_HIP(hipMemcpyAsync(b->d_slot_of.ptr, b->slot_of.data(), sizeof(int) * R, hipMemcpyHostToDevice, s));
@@ -563,6 +548,7 @@ extern "C" int hymd_batch_create(hymd_batch **out, int32_t n_replicas, const int
     HYMD_HIP(hipMemcpyAsync(b->d_row_slot.ptr, row_slot.data(), sizeof(int) * row_slot.size(), hipMemcpyHostToDevice,
                             s));
     HYMD_HIP(hipMemcpyAsync(b->d_row0.ptr, row0.data(), sizeof(int64_t) * R, hipMemcpyHostToDevice, s));
+    HYMD_HIP(hipMemcpyAsync(b->d_kf.ptr, kf.data(), sizeof(double2) * R, hipMemcpyHostToDevice, s));
     HYMD_TRY(zero_words(b->counts.ptr, rows + 2, s));
     HYMD_HIP(hipStreamSynchronize(s));
     *out = b.release();
@@ -591,9 +577,21 @@ static int batch_run(hymd_batch *b, const float *x, const int32_t *types, const 
         // the force stages' buffers are sized on first use
         HYMD_TRY(b->grad.reserve(sizeof(float2) * std::max<int64_t>(b->grad_total, 1)));
         HYMD_TRY(b->fgrid.reserve(sizeof(float) * std::max<int64_t>(b->fgrid_total, 1)));
-        double *hc = (double *)b->h_coupling.ptr;
-        for (int r = 0; r < R; ++r)
-            std::memcpy(hc + (int64_t)b->slot_of[r] * T * T, coupling + (int64_t)r * T * T, sizeof(double) * T * T);
+        size_t tmp = 0;
+        for (const auto &gp : b->groups)
+            tmp = std::max(tmp, (size_t)fft_yz_tmp(gp->plan, force_job(b, *gp)) * (size_t)b->geo[gp->first].gc);
+        if (tmp) HYMD_TRY(b->tmp.reserve(sizeof(float2) * tmp));
+        FieldK *hp = (FieldK *)b->h_par.ptr;
+        for (int r = 0; r < R; ++r) {
+            FieldK &p = hp[b->slot_of[r]];
+            p = FieldK{};
+            p.T = T;
+            p.sigma2 = sigma[r] * sigma[r];
+            p.inv_g = 1.0 / (double)b->geo[b->slot_of[r]].g;
+            for (int t = 0; t < T; ++t)
+                for (int u = 0; u < T; ++u)
+                    p.Af[t * HYMD_MAX_TYPES + u] = (float)coupling[((int64_t)r * T + t) * T + u];
+        }
     }
     hipStream_t s = b->stream;
     // inputs written on the caller's stream are ready before the batch reads them
@@ -601,8 +599,7 @@ static int batch_run(hymd_batch *b, const float *x, const int32_t *types, const 
     HYMD_HIP(hipStreamWaitEvent(s, b->ev_in, 0));
     HYMD_HIP(hipMemcpyAsync(b->d_sigma2.ptr, hs, sizeof(double) * R, hipMemcpyHostToDevice, s));
     if (forces)
-        HYMD_HIP(hipMemcpyAsync(b->d_coupling.ptr, b->h_coupling.ptr, sizeof(double) * T * T * R,
-                                hipMemcpyHostToDevice, s));
+        HYMD_HIP(hipMemcpyAsync(b->d_par.ptr, b->h_par.ptr, sizeof(FieldK) * R, hipMemcpyHostToDevice, s));
     if (use_graph) {
         if (!b->exec[gi] || b->cap_x[gi] != x || b->cap_types[gi] != types || (forces && b->cap_forces != forces)) {
             if (b->exec[gi]) {

@@ -17,6 +17,7 @@
 
 #include "fft.h"
 #include "field_dev.h"
+#include "xline.h"
 
 namespace hymd {
 
@@ -378,404 +379,18 @@ __global__ void __launch_bounds__(kBlock) readout_kernel(const float *__restrict
     }
 }
 
-struct FieldK {
-    int T;
-    int want_energy;
-    double sigma2;   // sigma^2
-    double inv_g;    // 1/G (r2c normalisation)
-    double c0;
-    double Ad[HYMD_MAX_TYPES * HYMD_MAX_TYPES];
-    double b[HYMD_MAX_TYPES];
-};
-
-// Input: spec[t] = unnormalised FFT of rho_t = paint_t/dV.  Outputs:
-// grad[3t+d] = -i k_d V_t(k), phif[t] = H rho_t/G (optional), spec[t] <-
-// V_t(k) (optional, in place), per-block energy partial sums.
+// The k-space pass by itself (field_dev.h::kspace_point): for more than 8
+// types, a one-stage x axis (Mx = 4), and where the spectra of all three
+// transforms are wanted first (the moments).
 template <int MAXT>
-__global__ void __launch_bounds__(kBlock) field_kspace_kernel(float2 *__restrict__ spec,
-                                                               float2 *__restrict__ grad,
-                                                               float2 *__restrict__ phif, int write_v, KGeom g,
-                                                               FieldK p, double *__restrict__ partials) {
+__global__ void __launch_bounds__(kBlock) field_kspace_kernel(const float2 *__restrict__ spec,
+                                                              float2 *__restrict__ out, float2 *__restrict__ phif,
+                                                              KGeom g, FieldK p, double *__restrict__ partials) {
     double e_acc[1] = {0.0};
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t kk = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; kk < g.gc; kk += stride) {
-        double k[3], kd[3], wgt;
-        kvec(g, kk, k, kd, wgt);
-        const double k2 = k[0] * k[0] + k[1] * k[1] + k[2] * k[2];
-        const float H = (float)exp(-0.5 * p.sigma2 * k2);
-        const float hn = (float)((double)H * p.inv_g);
-        float2 ph[MAXT];
-#pragma unroll
-        for (int t = 0; t < MAXT; ++t)
-            if (t < p.T) ph[t] = cscale(spec[(int64_t)t * g.gc + kk], hn);
-        if (phif) {
-#pragma unroll
-            for (int t = 0; t < MAXT; ++t)
-                if (t < p.T) phif[(int64_t)t * g.gc + kk] = ph[t];
-        }
-        if (p.want_energy) {
-            double e = 0.0;
-#pragma unroll
-            for (int t = 0; t < MAXT; ++t) {
-                if (t >= p.T) continue;
-#pragma unroll
-                for (int s = 0; s < MAXT; ++s) {
-                    if (s >= p.T) continue;
-                    e += 0.5 * p.Ad[t * HYMD_MAX_TYPES + s] *
-                         ((double)ph[t].x * (double)ph[s].x + (double)ph[t].y * (double)ph[s].y);
-                }
-            }
-            e *= wgt;
-            if (kk == 0) {
-                for (int t = 0; t < p.T; ++t) e += p.b[t] * (double)ph[t].x;
-                e += p.c0;
-            }
-            e_acc[0] += e;
-        }
-#pragma unroll
-        for (int t = 0; t < MAXT; ++t) {
-            if (t >= p.T) continue;
-            float2 v = make_float2(0.f, 0.f);
-#pragma unroll
-            for (int s = 0; s < MAXT; ++s)
-                if (s < p.T) {
-                    const float a = (float)p.Ad[t * HYMD_MAX_TYPES + s];
-                    v.x += a * ph[s].x;
-                    v.y += a * ph[s].y;
-                }
-            v = cscale(v, H);
-            if (kk == 0) v.x += (float)p.b[t];
-            // -i k_d v = (k_d v.y, -k_d v.x)
-            float2 *gt = grad + (int64_t)(3 * t) * g.gc + kk;
-            gt[0] = make_float2((float)kd[0] * v.y, -(float)kd[0] * v.x);
-            gt[g.gc] = make_float2((float)kd[1] * v.y, -(float)kd[1] * v.x);
-            gt[2 * g.gc] = make_float2((float)kd[2] * v.y, -(float)kd[2] * v.x);
-            if (write_v) spec[(int64_t)t * g.gc + kk] = v;
-        }
-    }
+    for (int64_t kk = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; kk < g.gc; kk += stride)
+        e_acc[0] += kspace_point<MAXT>(spec, out, phif, g, p, kk);
     if (partials) block_reduce_store<1>(e_acc, partials + blockIdx.x);
-}
-
-// Forward x pass fused with the k-space pass.  One workgroup owns W
-// consecutive (y, kz) lines of all T density spectra (after their z and y
-// passes): it runs their forward FFTs along x, then the k-space pass of
-// field_kspace_kernel at every k of those lines (same arithmetic, so the same
-// bits) and writes the 3T gradient spectra -i k_d V_t for the inverse passes,
-// so the T transformed spectra never make a round trip through HBM.  LDS:
-// twiddles, two buffers of T W lines.
-template <int MAXT>
-__global__ void __launch_bounds__(kBlock) field_xline_kernel(const float2 *__restrict__ spec,
-                                                              float2 *__restrict__ grad, KGeom g, FieldK p,
-                                                              FftAxis ax, const float2 *__restrict__ tw_glob,
-                                                              int wshift, double *__restrict__ partials) {
-    extern __shared__ float2 smem[];
-    const int n = ax.n;  // Mx
-    const int W = 1 << wshift;
-    const int T = p.T;
-    float2 *tw = smem;
-    float2 *A = tw + n;
-    float2 *B = A + T * W * ax.ld;
-    const int plane = g.my * g.zh;  // lines, and the element stride along x
-    const int line0 = (int)xcd_block(blockIdx.x, gridDim.x) * W;
-    const int wv = min(W, plane - line0);
-    for (int i = threadIdx.x; i < n - 1; i += blockDim.x) tw[i] = tw_glob[i];
-    // load T x W lines, W consecutive lines contiguous in memory
-    const int nel = T * W * n;
-    for (int i0 = threadIdx.x; i0 < nel; i0 += kBlock * kLoadBatch) {
-        float2 v[kLoadBatch];
-#pragma unroll
-        for (int j = 0; j < kLoadBatch; ++j) {
-            const int idx = i0 + j * kBlock;
-            v[j] = make_float2(0.f, 0.f);
-            if (idx < nel) {
-                const int l = idx & (W - 1), te = idx >> wshift, t = fdiv(te, ax.ndiv), e = te - t * n;
-                if (l < wv) v[j] = spec[(int64_t)t * g.gc + (int64_t)e * plane + line0 + l];
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < kLoadBatch; ++j) {
-            const int idx = i0 + j * kBlock;
-            if (idx < nel) {
-                const int l = idx & (W - 1), te = idx >> wshift, t = fdiv(te, ax.ndiv), e = te - t * n;
-                A[(t * W + l) * ax.ld + e] = v[j];
-            }
-        }
-    }
-    __syncthreads();
-    const float2 *F = fft_lds(A, B, T * W, ax, tw, -1.f);
-    // k-space pass, writing -i k_d V_t(k)
-    double e_acc[1] = {0.0};
-    for (int idx = threadIdx.x; idx < W * n; idx += blockDim.x) {
-        const int l = idx & (W - 1), e = idx >> wshift;
-        if (l >= wv) continue;
-        const int64_t kk = (int64_t)e * plane + line0 + l;
-        double k[3], kd[3], wgt;
-        kvec(g, kk, k, kd, wgt);
-        const double k2 = k[0] * k[0] + k[1] * k[1] + k[2] * k[2];
-        const float H = (float)exp(-0.5 * p.sigma2 * k2);
-        const float hn = (float)((double)H * p.inv_g);
-        float2 ph[MAXT];
-#pragma unroll
-        for (int t = 0; t < MAXT; ++t)
-            if (t < T) ph[t] = cscale(F[(t * W + l) * ax.ld + e], hn);
-        if (p.want_energy) {
-            double en = 0.0;
-#pragma unroll
-            for (int t = 0; t < MAXT; ++t) {
-                if (t >= T) continue;
-#pragma unroll
-                for (int u = 0; u < MAXT; ++u) {
-                    if (u >= T) continue;
-                    en += 0.5 * p.Ad[t * HYMD_MAX_TYPES + u] *
-                          ((double)ph[t].x * (double)ph[u].x + (double)ph[t].y * (double)ph[u].y);
-                }
-            }
-            en *= wgt;
-            if (kk == 0) {
-#pragma unroll
-                for (int t = 0; t < MAXT; ++t)
-                    if (t < T) en += p.b[t] * (double)ph[t].x;
-                en += p.c0;
-            }
-            e_acc[0] += en;
-        }
-#pragma unroll
-        for (int t = 0; t < MAXT; ++t) {
-            if (t >= T) continue;
-            float2 v = make_float2(0.f, 0.f);
-#pragma unroll
-            for (int u = 0; u < MAXT; ++u)
-                if (u < T) {
-                    const float a = (float)p.Ad[t * HYMD_MAX_TYPES + u];
-                    v.x += a * ph[u].x;
-                    v.y += a * ph[u].y;
-                }
-            v = cscale(v, H);
-            if (kk == 0) v.x += (float)p.b[t];
-            float2 *gt = grad + (int64_t)(3 * t) * g.gc + kk;
-            gt[0] = make_float2((float)kd[0] * v.y, -(float)kd[0] * v.x);
-            gt[g.gc] = make_float2((float)kd[1] * v.y, -(float)kd[1] * v.x);
-            gt[2 * g.gc] = make_float2((float)kd[2] * v.y, -(float)kd[2] * v.x);
-        }
-    }
-    if (partials) block_reduce_store<1>(e_acc, partials + blockIdx.x);
-}
-
-// Forward x pass, k-space pass and the inverse x passes in one workgroup.
-// k_y and k_z are constant along an x line, so the x-inverse of -i k_d V_t
-// for d = y, z is -i k_d times the x-inverse of V_t: per line and type only
-// two inverse transforms are needed, IFFT_x(-i k_x V_t) -> out[t] and
-// IFFT_x(V_t) -> out[T + t]; fft_c2r_yz_grad applies -i k_y / -i k_z in its
-// y-z plane pass.  The T spectra are transformed in place in one LDS buffer
-// of T W lines; V_t waits in registers (PMAX positions per thread) while the
-// x-gradient family is transformed and stored.
-// x-line geometry: runtime (Mx, W, T from the plan) or compile-time (Mx = N,
-// T types, W lines per workgroup), the latter with every index map a constant
-// multiply-shift and the Stockham stages of fft_inplace_ct.
-template <int ELEMS>
-struct XlineRt {
-    static constexpr bool kCt = false;
-    int n, W, wshift, T, ld;
-    FastDiv ndiv, flines;
-    FftAxis ax;
-    __device__ int div_n(int i) const { return fdiv(i, ndiv); }
-    template <int SGN, int NT>
-    __device__ void fft(float2 *D, const float2 *tw) const {
-        fft_inplace<ELEMS>(D, 1, ld, T * W, flines, ax, tw, (float)SGN);
-    }
-};
-
-template <int T_, int N, int W_>
-struct XlineCt {
-    static constexpr int n = N, W = W_, T = T_, ld = N + 1;
-    static constexpr int wshift = W_ == 1 ? 0 : W_ == 2 ? 1 : W_ == 4 ? 2 : W_ == 8 ? 3 : 4;
-    static constexpr bool kCt = true;
-    __device__ int div_n(int i) const { return i / N; }
-    template <int SGN, int NT>
-    __device__ void fft(float2 *D, const float2 *tw) const {
-        fft_inplace_ct<N, T_ * W_, 1, N + 1, NT, SGN>(D, tw);
-    }
-    // the same with the first stage's inputs from ld(line, e) / the last
-    // stage's outputs to st(line, e, value), line = t W + l
-    template <int SGN, int NT, class Load>
-    __device__ void fft_from(float2 *D, const float2 *tw, Load ld) const {
-        fft_first_ct<N, T_ * W_, 1, N + 1, NT, SGN>(D, ld);
-        fft_inplace_ct<N, T_ * W_, 1, N + 1, NT, SGN, 1>(D, tw);
-    }
-    template <int SGN, int NT, class Store>
-    __device__ void fft_to(float2 *D, const float2 *tw, Store st) const {
-        fft_inplace_ct<N, T_ * W_, 1, N + 1, NT, SGN, 0, CtPlan<N>::v.ns - 1>(D, tw);
-        fft_last_ct<N, T_ * W_, 1, N + 1, NT, SGN, false>(D, tw, st);
-    }
-};
-
-struct PmeK {
-    double sigma2;
-    double inv_g;
-    double four_pi_elec;  // 4 pi k_e / eps_r
-};
-
-// PME (T = 1): the k-space pass is pme_kspace_kernel's (psi = 4 pi elec H
-// rho~ / |k|^2 with the same FP64 arithmetic); outputs -i k_x psi and psi.
-template <int MAXT, int NT, class G, bool PME = false>
-__global__ void __launch_bounds__(NT) field_xline_grad_kernel(const float2 *__restrict__ spec,
-                                                              float2 *__restrict__ out, KGeom g, FieldK p, G geo,
-                                                              const float2 *__restrict__ tw_glob,
-                                                              double *__restrict__ partials, PmeK pk) {
-    constexpr int PMAX = 16 / MAXT;  // W n <= NT PMAX (checked on the host)
-    extern __shared__ float2 smem[];
-    const int n = geo.n;  // Mx
-    const int W = geo.W, wshift = geo.wshift;
-    const int T = geo.T;
-    const int ld = geo.ld;
-    float2 *tw = smem;
-    float2 *D = tw + n;  // line (t W + l) at D + (t W + l) ld
-    const int plane = g.my * g.zh;
-    const int line0 = (int)xcd_block(blockIdx.x, gridDim.x) * W;
-    const int wv = min(W, plane - line0);
-    for (int i = threadIdx.x; i < n - 1; i += NT) tw[i] = tw_glob[i];
-    const int nel = T * W * n;
-    if constexpr (G::kCt) {
-        // the forward transform's first stage reads the lines from global memory
-        geo.template fft_from<-1, NT>(D, tw, [&](int line, int e) -> float2 {
-            const int t = line >> wshift, l = line & (W - 1);
-            return l < wv ? spec[(int64_t)t * g.gc + (int64_t)e * plane + line0 + l] : make_float2(0.f, 0.f);
-        });
-    } else {
-    for (int i0 = threadIdx.x; i0 < nel; i0 += NT * kLoadBatch) {
-        float2 v[kLoadBatch];
-#pragma unroll
-        for (int j = 0; j < kLoadBatch; ++j) {
-            const int idx = i0 + j * NT;
-            v[j] = make_float2(0.f, 0.f);
-            if (idx < nel) {
-                const int l = idx & (W - 1), te = idx >> wshift, t = geo.div_n(te), e = te - t * n;
-                if (l < wv) v[j] = spec[(int64_t)t * g.gc + (int64_t)e * plane + line0 + l];
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < kLoadBatch; ++j) {
-            const int idx = i0 + j * NT;
-            if (idx < nel) {
-                const int l = idx & (W - 1), te = idx >> wshift, t = geo.div_n(te), e = te - t * n;
-                D[(t * W + l) * ld + e] = v[j];
-            }
-        }
-    }
-    __syncthreads();
-    geo.template fft<-1, NT>(D, tw);
-    }
-    // k-space pass (the arithmetic of field_kspace_kernel): V_t kept in
-    // registers, -i k_x V_t written back in place
-    double e_acc[1] = {0.0};
-    float2 hold[PMAX][MAXT];
-#pragma unroll
-    for (int j = 0; j < PMAX; ++j) {
-        const int pos = threadIdx.x + j * NT;
-        const int l = pos & (W - 1), e = pos >> wshift;
-        if (pos >= W * n || l >= wv) {
-#pragma unroll
-            for (int t = 0; t < MAXT; ++t) hold[j][t] = make_float2(0.f, 0.f);
-            continue;
-        }
-        const int64_t kk = (int64_t)e * plane + line0 + l;
-        double k[3], kd[3], wgt;
-        kvec(g, kk, k, kd, wgt);
-        if constexpr (PME) {
-            double k2 = k[0] * k[0] + k[1] * k[1] + k[2] * k[2];
-            const double H = exp(-0.5 * pk.sigma2 * k2);
-            if (kk == 0) k2 = 1.0;
-            const float2 sp = D[l * ld + e];
-            const double rx = (double)sp.x * pk.inv_g, ry = (double)sp.y * pk.inv_g;
-            const double f = pk.four_pi_elec * H / k2;
-            const double px = f * rx, py = f * ry;
-            e_acc[0] += 0.5 * wgt * (rx * px + ry * py);
-            hold[j][0] = make_float2((float)px, (float)py);
-            D[l * ld + e] = make_float2((float)(kd[0] * py), (float)(-kd[0] * px));
-            continue;
-        }
-        const double k2 = k[0] * k[0] + k[1] * k[1] + k[2] * k[2];
-        const float H = (float)exp(-0.5 * p.sigma2 * k2);
-        const float hn = (float)((double)H * p.inv_g);
-        float2 ph[MAXT];
-#pragma unroll
-        for (int t = 0; t < MAXT; ++t) ph[t] = t < T ? cscale(D[(t * W + l) * ld + e], hn) : make_float2(0.f, 0.f);
-        if (p.want_energy) {
-            double en = 0.0;
-#pragma unroll
-            for (int t = 0; t < MAXT; ++t) {
-                if (t >= T) continue;
-#pragma unroll
-                for (int u = 0; u < MAXT; ++u) {
-                    if (u >= T) continue;
-                    en += 0.5 * p.Ad[t * HYMD_MAX_TYPES + u] *
-                          ((double)ph[t].x * (double)ph[u].x + (double)ph[t].y * (double)ph[u].y);
-                }
-            }
-            en *= wgt;
-            if (kk == 0) {
-#pragma unroll
-                for (int t = 0; t < MAXT; ++t)
-                    if (t < T) en += p.b[t] * (double)ph[t].x;
-                en += p.c0;
-            }
-            e_acc[0] += en;
-        }
-        const float kx = (float)kd[0];
-#pragma unroll
-        for (int t = 0; t < MAXT; ++t) {
-            float2 v = make_float2(0.f, 0.f);
-#pragma unroll
-            for (int u = 0; u < MAXT; ++u)
-                if (u < T) {
-                    const float a = (float)p.Ad[t * HYMD_MAX_TYPES + u];
-                    v.x += a * ph[u].x;
-                    v.y += a * ph[u].y;
-                }
-            v = cscale(v, H);
-            if (kk == 0) v.x += (float)p.b[t];
-            hold[j][t] = v;
-            if (t < T) D[(t * W + l) * ld + e] = make_float2(kx * v.y, -kx * v.x);
-        }
-    }
-    __syncthreads();
-    if constexpr (G::kCt) {
-        // the inverse transforms' last stage writes the lines to global memory
-        geo.template fft_to<1, NT>(D, tw, [&](int line, int e, float2 v) {
-            const int t = line >> wshift, l = line & (W - 1);
-            if (l < wv) out[(int64_t)t * g.gc + (int64_t)e * plane + line0 + l] = v;
-        });
-    } else {
-        geo.template fft<1, NT>(D, tw);
-        for (int idx = threadIdx.x; idx < nel; idx += NT) {
-            const int l = idx & (W - 1), te = idx >> wshift, t = geo.div_n(te), e = te - t * n;
-            if (l < wv) out[(int64_t)t * g.gc + (int64_t)e * plane + line0 + l] = D[(t * W + l) * ld + e];
-        }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < PMAX; ++j) {
-        const int pos = threadIdx.x + j * NT;
-        if (pos >= W * n) continue;
-        const int l = pos & (W - 1), e = pos >> wshift;
-#pragma unroll
-        for (int t = 0; t < MAXT; ++t)
-            if (t < T) D[(t * W + l) * ld + e] = hold[j][t];
-    }
-    __syncthreads();
-    if constexpr (G::kCt) {
-        geo.template fft_to<1, NT>(D, tw, [&](int line, int e, float2 v) {
-            const int t = line >> wshift, l = line & (W - 1);
-            if (l < wv) out[(int64_t)(T + t) * g.gc + (int64_t)e * plane + line0 + l] = v;
-        });
-    } else {
-        geo.template fft<1, NT>(D, tw);
-        for (int idx = threadIdx.x; idx < nel; idx += NT) {
-            const int l = idx & (W - 1), te = idx >> wshift, t = geo.div_n(te), e = te - t * n;
-            if (l < wv) out[(int64_t)(T + t) * g.gc + (int64_t)e * plane + line0 + l] = D[(t * W + l) * ld + e];
-        }
-    }
-    if (partials) block_reduce_store<1, NT>(e_acc, partials + blockIdx.x);
 }
 
 // Spectral moments (P, Q, phi~(0)) of the filtered densities, one partial
@@ -953,15 +568,12 @@ __global__ void __launch_bounds__(kBlock) field_pressure_kernel(const float2 *__
 }
 
 
-// PME (field.py:363-397): rho~ = H rho/G; psi = 4 pi elec rho~/|k|^2 (|k|^2 := 1
-// at k = 0); E_d = -i k_d psi.  Energy partials: 1/2 wgt Re(rho^* psi).
-// grad_form: out[0] = -i k_x psi, out[1] = psi (the inputs of the x-inverse
-// and fft_c2r_yz_grad, which applies -i k_y and -i k_z); otherwise out[d] =
-// E_d and, with write_psi, out[3] = psi.
+// PME (field.py:363-397) by itself, for a one-stage x axis (Mx = 4): rho~ = H
+// rho/G; psi = 4 pi elec rho~/|k|^2 (|k|^2 := 1 at k = 0); out[0] = -i k_x psi,
+// out[1] = psi.  Energy partials: 1/2 wgt Re(rho^* psi).
 __global__ void __launch_bounds__(kBlock) pme_kspace_kernel(const float2 *__restrict__ spec,
-                                                             float2 *__restrict__ out, int write_psi,
-                                                             int grad_form, KGeom g, PmeK p,
-                                                             double *__restrict__ partials) {
+                                                            float2 *__restrict__ out, KGeom g, PmeK p,
+                                                            double *__restrict__ partials) {
     double e_acc[1] = {0.0};
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     for (int64_t kk = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; kk < g.gc; kk += stride) {
@@ -976,13 +588,7 @@ __global__ void __launch_bounds__(kBlock) pme_kspace_kernel(const float2 *__rest
         const double px = f * rx, py = f * ry;                                // psi
         e_acc[0] += 0.5 * wgt * (rx * px + ry * py);
         out[kk] = make_float2((float)(kd[0] * py), (float)(-kd[0] * px));
-        if (grad_form) {
-            out[g.gc + kk] = make_float2((float)px, (float)py);
-            continue;
-        }
-        out[g.gc + kk] = make_float2((float)(kd[1] * py), (float)(-kd[1] * px));
-        out[2 * g.gc + kk] = make_float2((float)(kd[2] * py), (float)(-kd[2] * px));
-        if (write_psi) out[3 * g.gc + kk] = make_float2((float)px, (float)py);
+        out[g.gc + kk] = make_float2((float)px, (float)py);
     }
     if (partials) block_reduce_store<1>(e_acc, partials + blockIdx.x);
 }
@@ -1045,7 +651,8 @@ struct hymd_pm {
     DevBuf paint;     // max_types x G: float densities, or int64 for the accumulate-mode paint
     DevBuf spec;      // max_types x Gc complex
     DevBuf grad;      // max(3 max_types, 4) x Gc complex
-    DevBuf cscratch;  // max_types x Gc complex (phi / v_ext inverse transforms)
+    DevBuf cscratch;  // complex scratch of the line passes (and of hymd_fft_c2r)
+    DevBuf phix;      // x-inverse filtered spectra, when the densities are asked for
     DevBuf rscratch;  // 3 x G float (PME field when the caller passes none)
     DevBuf partials;  // energy partial sums
     DevBuf result;    // reduced doubles
@@ -1071,7 +678,7 @@ struct hymd_pm {
 
 uint64_t hymd::pm_generation(const hymd_pm *pm) {
     uint64_t g = pm->box_version;
-    for (const DevBuf *b : {&pm->paint, &pm->spec, &pm->grad, &pm->cscratch, &pm->rscratch, &pm->partials,
+    for (const DevBuf *b : {&pm->paint, &pm->spec, &pm->grad, &pm->cscratch, &pm->phix, &pm->rscratch, &pm->partials,
                             &pm->result, &pm->mpart, &pm->keys, &pm->perm, &pm->xs, &pm->ws, &pm->counts,
                             &pm->start, &pm->tiles})
         g += b->allocs;
@@ -1085,175 +692,6 @@ int hymd::pm_clone(const hymd_pm *src, int32_t max_types, void *stream, hymd_pm 
 
 void hymd::pm_box(const hymd_pm *pm, double box[3]) {
     for (int d = 0; d < 3; ++d) box[d] = pm->mesh.box[d];
-}
-
-// LDS budget of one x-line workgroup (two per CU)
-constexpr size_t kXlineLdsBytes = 80 * 1024;
-
-static size_t xline_lds(const FftPlan &f, int T, int W) {
-    return sizeof(float2) * ((size_t)f.ax.n + 2 * (size_t)T * W * f.ax.ld);
-}
-
-// Lines per x-line workgroup for T types (0: the fused pass does not fit).
-static int xline_width(const FftPlan &f, int T) {
-    for (int W = 16; W >= 2; W >>= 1)
-        if (xline_lds(f, T, W) <= kXlineLdsBytes) return W;
-    return 0;
-}
-
-template <int MAXT>
-static int launch_xline(hymd_pm *pm, const float2 *spec, float2 *grad, const KGeom &g, const FieldK &p, int W,
-                        double *partials, int *nblocks) {
-    const FftPlan &f = pm->fft;
-    const int plane = g.my * g.zh;
-    const int nb = (plane + W - 1) / W;
-    const size_t lds = xline_lds(f, p.T, W);
-    static bool attr_set = false;  // the opt-in is per kernel and process
-    if (!attr_set && lds > 64 * 1024) {
-        HYMD_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&field_xline_kernel<MAXT>),
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)kXlineLdsBytes));
-        attr_set = true;
-    }
-    int wshift = 0;
-    while ((1 << wshift) < W) ++wshift;
-    field_xline_kernel<MAXT><<<nb, kBlock, lds, pm->stream>>>(spec, grad, g, p, f.ax, (const float2 *)f.tw_x.ptr,
-                                                              wshift, partials);
-    HYMD_HIP(hipGetLastError());
-    *nblocks = nb;
-    return HYMD_OK;
-}
-
-constexpr int kXlineGradThreads = 256;
-constexpr int kXlineGradElems = 16;  // values per thread and in-place stage
-// Workgroups of 512 or 1024 threads (one per CU at up to 150 KB of LDS) for
-// long x lines with many types, where 256 threads hold only 2 lines: a
-// workgroup's lines are neighbouring (y, k_z) columns, so W lines give W * 8
-// contiguous bytes per x row, and at 16 bytes the partial HBM bursts double
-// the traffic of the pass.
-constexpr size_t kXlineWideLdsBytes = 150 * 1024;
-
-struct XlineShape {
-    int W = 0, NT = kXlineGradThreads;
-};
-
-// Lines per workgroup W of field_xline_grad_kernel with NT threads for T
-// types: the registers hold PMAX positions per thread (W n <= NT PMAX), the
-// in-place stages kXlineGradElems values per thread, LDS the T W lines.
-static bool xline_grad_fits(const FftPlan &f, int T, int W, int NT) {
-    const int pmax = 16 / moments_maxt(T);
-    if ((int64_t)W * f.ax.n > (int64_t)NT * pmax) return false;
-    const size_t lim = NT == kXlineGradThreads ? kXlineLdsBytes : kXlineWideLdsBytes;
-    if (sizeof(float2) * ((size_t)f.ax.n + (size_t)T * W * f.ax.ld) > lim) return false;
-    return fft_inplace_fits(f.ax, T * W, NT, kXlineGradElems);
-}
-
-// The x-line shape: `want` lines with the fewest threads that fit it, else
-// the widest W that fits 256 threads when that is at least 4 lines, else 8
-// or 16 lines with 512 or 1024 threads, else 2 lines (W = 0: the fused pass
-// does not fit).
-static XlineShape xline_grad_shape(const FftPlan &f, int T, int want = 0) {
-    const int nts[3] = {kXlineGradThreads, 2 * kXlineGradThreads, 4 * kXlineGradThreads};
-    if (want > 0)
-        for (int NT : nts)
-            if (xline_grad_fits(f, T, want, NT)) return XlineShape{want, NT};
-    for (int W = 16; W >= 4; W >>= 1)
-        if (xline_grad_fits(f, T, W, kXlineGradThreads)) return XlineShape{W, kXlineGradThreads};
-    for (int W = 16; W >= 8; W >>= 1)
-        for (int NT : {2 * kXlineGradThreads, 4 * kXlineGradThreads})
-            if (xline_grad_fits(f, T, W, NT)) return XlineShape{W, NT};
-    if (xline_grad_fits(f, T, 2, kXlineGradThreads)) return XlineShape{2, kXlineGradThreads};
-    return XlineShape{};
-}
-
-template <int MAXT, int NT, class G>
-static int launch_xline_grad_g(hymd_pm *pm, const float2 *spec, float2 *out, const KGeom &g, const FieldK &p, int W,
-                               const G &geo, double *partials, int *nblocks, const PmeK *pme) {
-    const FftPlan &f = pm->fft;
-    const int plane = g.my * g.zh;
-    const int nb = (plane + W - 1) / W;
-    const size_t lds = sizeof(float2) * ((size_t)f.ax.n + (size_t)p.T * W * f.ax.ld);
-    const size_t lim = NT == kXlineGradThreads ? kXlineLdsBytes : kXlineWideLdsBytes;
-    static bool attr_set = false;  // the opt-in is per kernel and process
-    if (!attr_set && lds > 64 * 1024) {
-        HYMD_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&field_xline_grad_kernel<MAXT, NT, G>),
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lim));
-        HYMD_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&field_xline_grad_kernel<MAXT, NT, G, true>),
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lim));
-        attr_set = true;
-    }
-    if (pme)
-        field_xline_grad_kernel<MAXT, NT, G, true><<<nb, NT, lds, pm->stream>>>(
-            spec, out, g, p, geo, (const float2 *)f.tw_x.ptr, partials, *pme);
-    else
-        field_xline_grad_kernel<MAXT, NT, G><<<nb, NT, lds, pm->stream>>>(spec, out, g, p, geo,
-                                                                          (const float2 *)f.tw_x.ptr, partials, PmeK{});
-    HYMD_HIP(hipGetLastError());
-    *nblocks = nb;
-    return HYMD_OK;
-}
-
-template <int MAXT, class G>
-static int launch_xline_grad_nt(hymd_pm *pm, const float2 *spec, float2 *out, const KGeom &g, const FieldK &p,
-                                const XlineShape &sh, const G &geo, double *partials, int *nblocks,
-                                const PmeK *pme) {
-    if (sh.NT == 4 * kXlineGradThreads)
-        return launch_xline_grad_g<MAXT, 4 * kXlineGradThreads>(pm, spec, out, g, p, sh.W, geo, partials, nblocks,
-                                                                pme);
-    if (sh.NT == 2 * kXlineGradThreads)
-        return launch_xline_grad_g<MAXT, 2 * kXlineGradThreads>(pm, spec, out, g, p, sh.W, geo, partials, nblocks,
-                                                                pme);
-    return launch_xline_grad_g<MAXT, kXlineGradThreads>(pm, spec, out, g, p, sh.W, geo, partials, nblocks, pme);
-}
-
-template <int N>
-static bool xline_ct_plan(const FftPlan &f) {
-    const StagePlan &sp = CtPlan<N>::v;
-    if (f.ax.n != N || f.ax.ld != N + 1 || f.ax.nstages != sp.ns) return false;
-    for (int i = 0; i < sp.ns; ++i)
-        if (f.ax.radix[i] != sp.r[i] || f.ax.twoff[i] != sp.twoff[i]) return false;
-    return true;
-}
-
-// The x-line pass for T types in the shape sh: a compile-time geometry for
-// Mx = 128 or 160 at the 256-thread W that xline_grad_shape picks there (run
-// at 512 threads for Mx = 128) and for Mx = 256 with six types at 8 lines of
-// 1024 threads or 4 of 512, the runtime one otherwise.
-static int launch_xline_grad(hymd_pm *pm, const float2 *spec, float2 *out, const KGeom &g, const FieldK &p,
-                             const XlineShape &sh, double *partials, int *nblocks, const PmeK *pme = nullptr) {
-    const FftPlan &f = pm->fft;
-    const int T = p.T, W = sh.W;
-    // NTH threads per workgroup for the 256-thread shape's lines and LDS: the
-    // Mx = 128 geometries run at 512, twice the waves in flight (the 128^3,
-    // T = 4 pass 33.6 -> 29.8 us); at 160 that made the peptide step slower
-#define HYMD_XLINE_CT(NX, TT, WW, MT, NTH)                                                                 \
-    if (sh.NT == kXlineGradThreads && f.ax.n == NX && T == TT && W == WW && xline_ct_plan<NX>(f))          \
-        return launch_xline_grad_g<MT, NTH>(pm, spec, out, g, p, W, XlineCt<TT, NX, WW>{}, partials, nblocks, pme);
-    HYMD_XLINE_CT(128, 1, 16, 2, 2 * kXlineGradThreads)
-    HYMD_XLINE_CT(128, 2, 16, 2, 2 * kXlineGradThreads)
-    HYMD_XLINE_CT(128, 3, 8, 4, 2 * kXlineGradThreads)
-    HYMD_XLINE_CT(128, 4, 8, 4, 2 * kXlineGradThreads)
-    HYMD_XLINE_CT(160, 1, 8, 2, kXlineGradThreads)
-    HYMD_XLINE_CT(160, 2, 8, 2, kXlineGradThreads)
-    HYMD_XLINE_CT(160, 3, 4, 4, kXlineGradThreads)
-    HYMD_XLINE_CT(160, 4, 4, 4, kXlineGradThreads)
-    HYMD_XLINE_CT(256, 1, 8, 2, kXlineGradThreads)
-#undef HYMD_XLINE_CT
-    // 256-point lines with six types (the 256^3 workloads): 8 lines of 1024
-    // threads or 4 lines of 512
-    if (f.ax.n == 256 && T == 6 && xline_ct_plan<256>(f)) {
-        if (sh.NT == 4 * kXlineGradThreads && W == 8)
-            return launch_xline_grad_g<8, 4 * kXlineGradThreads>(pm, spec, out, g, p, W, XlineCt<6, 256, 8>{},
-                                                                 partials, nblocks, pme);
-        if (sh.NT == 2 * kXlineGradThreads && W == 4)
-            return launch_xline_grad_g<8, 2 * kXlineGradThreads>(pm, spec, out, g, p, W, XlineCt<6, 256, 4>{},
-                                                                 partials, nblocks, pme);
-    }
-    int wshift = 0;
-    while ((1 << wshift) < W) ++wshift;
-    const XlineRt<kXlineGradElems> geo{f.ax.n, W, wshift, T, f.ax.ld, f.ax.ndiv, make_fastdiv((uint32_t)(T * W)), f.ax};
-    if (T <= 2) return launch_xline_grad_nt<2>(pm, spec, out, g, p, sh, geo, partials, nblocks, pme);
-    if (T <= 4) return launch_xline_grad_nt<4>(pm, spec, out, g, p, sh, geo, partials, nblocks, pme);
-    return launch_xline_grad_nt<8>(pm, spec, out, g, p, sh, geo, partials, nblocks, pme);
 }
 
 // LDS budget of one row-paint workgroup (int64 accumulators of tc types x Mz)
@@ -1311,9 +749,9 @@ extern "C" int hymd_pm_create(hymd_pm **out, const int32_t mesh[3], const double
     if (st == HYMD_OK) st = pm->paint.reserve(sizeof(int64_t) * m.g * max_types);
     if (st == HYMD_OK) st = pm->spec.reserve(sizeof(float2) * m.gc * max_types);
     if (st == HYMD_OK) st = pm->grad.reserve(sizeof(float2) * m.gc * std::max(3 * max_types, 4));
-    // energy partial rows: k-space blocks or x-line blocks (at least 2 lines each)
+    // energy partial rows: k-space blocks or x-line blocks (at least one line each)
     if (st == HYMD_OK)
-        st = pm->partials.reserve(sizeof(double) * (std::max<int64_t>(pm->kblocks, (int64_t)m.my * m.zh / 2 + 1) + 16));
+        st = pm->partials.reserve(sizeof(double) * (std::max<int64_t>(pm->kblocks, (int64_t)m.my * m.zh) + 16));
     if (st == HYMD_OK) st = pm->result.reserve(sizeof(double) * 16);
     if (st == HYMD_OK) st = pm->host.reserve(sizeof(double) * 16);
     if (st == HYMD_OK) st = pm->counts.reserve(sizeof(int) * (m.g + 2));
@@ -1407,7 +845,10 @@ static FieldK field_params(int T, const double *coupling, const double *shift, d
     p.c0 = constant;
     for (int t = 0; t < HYMD_MAX_TYPES; ++t) {
         p.b[t] = (shift && t < T) ? shift[t] : 0.0;
-        for (int u = 0; u < HYMD_MAX_TYPES; ++u) p.Ad[t * HYMD_MAX_TYPES + u] = (t < T && u < T) ? coupling[t * T + u] : 0.0;
+        for (int u = 0; u < HYMD_MAX_TYPES; ++u) {
+            p.Ad[t * HYMD_MAX_TYPES + u] = (t < T && u < T) ? coupling[t * T + u] : 0.0;
+            p.Af[t * HYMD_MAX_TYPES + u] = (float)p.Ad[t * HYMD_MAX_TYPES + u];
+        }
     }
     return p;
 }
@@ -1590,6 +1031,68 @@ extern "C" int hymd_readout(hymd_pm *pm, const float *grid, const float *x, int6
     return HYMD_OK;
 }
 
+// The y-z passes of the x-inverse spectra that kspace_pass left in pm->grad:
+// the force grids, optionally the potentials v and, from phix, the densities.
+static int yz_passes(hymd_pm *pm, int T, float *force_mesh, float *v, const float2 *phix, float *phi) {
+    const KGeom g = kgeom(pm);
+    YzJob job;
+    job.T = T;
+    job.in = (const float2 *)pm->grad.ptr;
+    job.in2 = phix;
+    job.force = force_mesh;
+    job.real_v = v;
+    job.real2 = phi;
+    job.kfy = g.kfac[1];
+    job.kfz = g.kfac[2];
+    const int tmp = fft_yz_tmp(pm->fft, job);
+    if (tmp) HYMD_TRY(pm->cscratch.reserve(sizeof(float2) * pm->mesh.gc * tmp));
+    return fft_yz_multi(pm->fft, job, (float2 *)pm->cscratch.ptr, pm->stream);
+}
+
+// The x transforms and the k-space pass of p.T types from the spectra in
+// pm->spec (after their z and y passes, or with `transformed` after all
+// three): pm->grad <- IFFT_x(-i k_x V_t), IFFT_x(V_t); optionally the filtered
+// spectra phif, their x-inverse phix and energy partials (*nblocks of them).
+// fused = false: as separate passes, the batched replicas' arithmetic.
+static int kspace_pass(hymd_pm *pm, const FieldK &p, bool transformed, float2 *phif, float2 *phix, double *partials,
+                       int *nblocks, bool fused = true) {
+    const Mesh &m = pm->mesh;
+    const int T = p.T;
+    hipStream_t s = pm->stream;
+    XlineJob job;
+    job.T = T;
+    job.spec = (const float2 *)pm->spec.ptr;
+    job.transformed = transformed;
+    job.out = (float2 *)pm->grad.ptr;
+    job.phif = phif;
+    job.phix = phix;
+    job.g = kgeom(pm);
+    job.p = p;
+    job.partials = partials;
+    const XlineShape sh = xline_shape(pm->fft, T, pm->xline_w, !phif && !phix && !transformed);
+    // 4 T half spectra written in runs of 32 bytes: from 256 x points on they
+    // cost more than the separate passes (256^3, six types, with densities and
+    // spectra 4333 against 3022 us; 200^3 1533 against 1587, 144^3, eight types
+    // 797 against 768; 8 lines, 256^3, four types 1900 against 2045)
+    const bool narrow = (phif || phix) && sh.W < 8 && m.mx >= 256;
+    if (sh.W > 0 && fused && !narrow) return xline_pass(pm->fft, sh, job, nblocks, s);
+    if (!transformed) HYMD_TRY(fft_forward_x(pm->fft, (float2 *)pm->spec.ptr, T, s));
+    if (phix && !phif) phif = phix;
+    if (T <= 4)
+        field_kspace_kernel<4><<<pm->kblocks, kBlock, 0, s>>>(job.spec, job.out, phif, job.g, p, partials);
+    else if (T <= 8)
+        field_kspace_kernel<8><<<pm->kblocks, kBlock, 0, s>>>(job.spec, job.out, phif, job.g, p, partials);
+    else
+        field_kspace_kernel<16><<<pm->kblocks, kBlock, 0, s>>>(job.spec, job.out, phif, job.g, p, partials);
+    HYMD_HIP(hipGetLastError());
+    *nblocks = pm->kblocks;
+    HYMD_TRY(fft_inverse_x(pm->fft, job.out, 2 * T, s));
+    if (!phix) return HYMD_OK;
+    if (phix != phif)
+        HYMD_HIP(hipMemcpyAsync(phix, phif, sizeof(float2) * m.gc * T, hipMemcpyDeviceToDevice, s));
+    return fft_inverse_x(pm->fft, phix, T, s);
+}
+
 static int update_field_impl(hymd_pm *pm, const float *x, const int32_t *types, int64_t n, int32_t n_types,
                              const double *coupling, const double *shift, double constant, const double *mass,
                              double sigma, float *force_mesh, float *phi, void *phi_fourier, float *v_ext,
@@ -1604,7 +1107,6 @@ static int update_field_impl(hymd_pm *pm, const float *x, const int32_t *types, 
     hipStream_t s = pm->stream;
     unsigned long long *grid = (unsigned long long *)pm->paint.ptr;
     float2 *spec = (float2 *)pm->spec.ptr;
-    float2 *grad = (float2 *)pm->grad.ptr;
 
     // 1. cell sort + gather paint of rho_t = paint_t / dV (float grids)
     float *rho = (float *)grid;  // the handle's paint buffer holds T float grids here
@@ -1612,85 +1114,19 @@ static int update_field_impl(hymd_pm *pm, const float *x, const int32_t *types, 
     HYMD_TRY(paint_sorted(pm, T, mass, rho, nullptr));
     FieldK p = field_params(T, coupling, shift, constant, sigma, m);
     p.want_energy = energy ? 1 : 0;
-    KGeom g0 = kgeom(pm);
-    const XlineShape sh = T <= 8 ? xline_grad_shape(pm->fft, T, pm->xline_w) : XlineShape{};
-    if (!phi && !phi_fourier && !v_ext && sh.W > 0) {
-        // force grids only: z + y forward passes; one pass for the forward x
-        // transform, the k-space pass and the 2T inverse x transforms; the
-        // y-z plane pass writes the 3T force grids
-        HYMD_TRY(fft_r2c_zy(pm->fft, rho, spec, T, s));
-        double *part = energy ? (double *)pm->partials.ptr : nullptr;
-        int nb = 0;
-        HYMD_TRY(launch_xline_grad(pm, spec, grad, g0, p, sh, part, &nb));
-        if (pm->fft.lds_plane) {
-            HYMD_TRY(fft_c2r_yz_grad(pm->fft, grad, force_mesh, T, g0.kfac[1], g0.kfac[2], 1.f, s));
-        } else {  // y-z planes too large for LDS: the y and z line passes
-            HYMD_TRY(pm->cscratch.reserve(sizeof(float2) * m.gc * 3 * T));
-            HYMD_TRY(fft_c2r_lines_grad(pm->fft, grad, (float2 *)pm->cscratch.ptr, force_mesh, T, g0.kfac[1],
-                                        g0.kfac[2], 1.f, s));
-        }
-        if (energy) {
-            double e = 0.0;
-            HYMD_TRY(read_result(pm, nb, 1, &e));
-            *energy = e * (m.box[0] * m.box[1] * m.box[2]);
-        }
-        return HYMD_OK;
-    }
-    const int W = xline_width(pm->fft, T);
-    if (!phi && !phi_fourier && !v_ext && W > 0) {
-        // force grids only: z + y forward passes, the forward x pass fused
-        // with the k-space pass, then the inverse x, y and z passes
-        HYMD_TRY(fft_r2c_zy(pm->fft, rho, spec, T, s));
-        double *part = energy ? (double *)pm->partials.ptr : nullptr;
-        int nb = 0;
-        if (T <= 4) HYMD_TRY(launch_xline<4>(pm, spec, grad, g0, p, W, part, &nb));
-        else if (T <= 8) HYMD_TRY(launch_xline<8>(pm, spec, grad, g0, p, W, part, &nb));
-        else HYMD_TRY(launch_xline<16>(pm, spec, grad, g0, p, W, part, &nb));
-        HYMD_TRY(fft_c2r(pm->fft, grad, force_mesh, 3 * T, 1.f, s));
-        if (energy) {
-            double e = 0.0;
-            HYMD_TRY(read_result(pm, nb, 1, &e));
-            *energy = e * (m.box[0] * m.box[1] * m.box[2]);
-        }
-        return HYMD_OK;
-    }
-    // 2. r2c
-    HYMD_TRY(fft_r2c_real(pm->fft, rho, spec, T, s));
-    // 3. fused filter / W' / filter / gradient
-    float2 *phif = (float2 *)phi_fourier;
-    if (phi && !phif) {
-        HYMD_TRY(pm->cscratch.reserve(sizeof(float2) * m.gc * T));
-        phif = (float2 *)pm->cscratch.ptr;
-    }
-    KGeom g = kgeom(pm);
-    double *partials = energy ? (double *)pm->partials.ptr : nullptr;
-    const int kb = pm->kblocks;
-    if (T <= 4)
-        field_kspace_kernel<4><<<kb, kBlock, 0, s>>>(spec, grad, phif, v_ext ? 1 : 0, g, p, partials);
-    else if (T <= 8)
-        field_kspace_kernel<8><<<kb, kBlock, 0, s>>>(spec, grad, phif, v_ext ? 1 : 0, g, p, partials);
-    else
-        field_kspace_kernel<16><<<kb, kBlock, 0, s>>>(spec, grad, phif, v_ext ? 1 : 0, g, p, partials);
-    HYMD_HIP(hipGetLastError());
-    // 4. force grids
-    HYMD_TRY(fft_c2r(pm->fft, grad, force_mesh, 3 * T, 1.f, s));
-    // 5. optional real-space outputs
-    if (v_ext) {
-        HYMD_TRY(fft_c2r(pm->fft, spec, v_ext, T, 1.f, s));
-    }
+    // 2. z + y forward passes; the x-line pass; the y-z pass writes the grids
+    HYMD_TRY(fft_r2c_zy(pm->fft, rho, spec, T, s));
+    float2 *phix = nullptr;
     if (phi) {
-        float2 *work = phif;
-        if (phi_fourier) {  // keep the caller's spectra intact
-            HYMD_TRY(pm->cscratch.reserve(sizeof(float2) * m.gc * T));
-            HYMD_HIP(hipMemcpyAsync(pm->cscratch.ptr, phi_fourier, sizeof(float2) * m.gc * T,
-                                    hipMemcpyDeviceToDevice, s));
-            work = (float2 *)pm->cscratch.ptr;
-        }
-        HYMD_TRY(fft_c2r(pm->fft, work, phi, T, 1.f, s));
+        HYMD_TRY(pm->phix.reserve(sizeof(float2) * m.gc * T));
+        phix = (float2 *)pm->phix.ptr;
     }
+    int nb = 0;
+    HYMD_TRY(kspace_pass(pm, p, false, (float2 *)phi_fourier, phix, energy ? (double *)pm->partials.ptr : nullptr, &nb));
+    HYMD_TRY(yz_passes(pm, T, force_mesh, v_ext, phix, phi));
     if (energy) {
         double e = 0.0;
-        HYMD_TRY(read_result(pm, kb, 1, &e));
+        HYMD_TRY(read_result(pm, nb, 1, &e));
         *energy = e * (m.box[0] * m.box[1] * m.box[2]);
     }
     return HYMD_OK;
@@ -1793,14 +1229,10 @@ extern "C" int hymd_field_moments(hymd_pm *pm, const float *x, const int32_t *ty
     HYMD_TRY(reduce_partials((const double *)part.ptr, nb, row, (double *)pm->result.ptr, s));
     HYMD_HIP(hipMemcpyAsync(pm->host.ptr, pm->result.ptr, sizeof(double) * row, hipMemcpyDeviceToHost, s));
     if (force_mesh) {
-        FieldK p = field_params(T, coupling, shift, 0.0, sigma, m);
-        float2 *grad = (float2 *)pm->grad.ptr;
-        if (T <= 4)
-            field_kspace_kernel<4><<<pm->kblocks, kBlock, 0, s>>>(spec, grad, nullptr, 0, g, p, nullptr);
-        else
-            field_kspace_kernel<8><<<pm->kblocks, kBlock, 0, s>>>(spec, grad, nullptr, 0, g, p, nullptr);
-        HYMD_HIP(hipGetLastError());
-        HYMD_TRY(fft_c2r(pm->fft, grad, force_mesh, 3 * T, 1.f, s));
+        int unused = 0;
+        HYMD_TRY(kspace_pass(pm, field_params(T, coupling, shift, 0.0, sigma, m), true, nullptr, nullptr, nullptr,
+                             &unused, false));
+        HYMD_TRY(yz_passes(pm, T, force_mesh, nullptr, nullptr, nullptr));
     }
     HYMD_HIP(hipStreamSynchronize(s));
     for (int j = 0; j < nv; ++j) moments[j] = ((double *)pm->host.ptr)[j];
@@ -1820,16 +1252,9 @@ extern "C" int hymd_field_forces_held(hymd_pm *pm, int32_t n_types, const double
                  "no density spectra of %d types are held (call hymd_field_moments first)", n_types);
     const Mesh &m = pm->mesh;
     const int T = n_types;
-    hipStream_t s = pm->stream;
-    FieldK p = field_params(T, coupling, shift, 0.0, sigma, m);
-    float2 *grad = (float2 *)pm->grad.ptr;
-    KGeom g = kgeom(pm);
-    if (T <= 4)
-        field_kspace_kernel<4><<<pm->kblocks, kBlock, 0, s>>>((float2 *)pm->spec.ptr, grad, nullptr, 0, g, p, nullptr);
-    else
-        field_kspace_kernel<8><<<pm->kblocks, kBlock, 0, s>>>((float2 *)pm->spec.ptr, grad, nullptr, 0, g, p, nullptr);
-    HYMD_HIP(hipGetLastError());
-    HYMD_TRY(fft_c2r(pm->fft, grad, force_mesh, 3 * T, 1.f, s));
+    int unused = 0;
+    HYMD_TRY(kspace_pass(pm, field_params(T, coupling, shift, 0.0, sigma, m), true, nullptr, nullptr, nullptr, &unused));
+    HYMD_TRY(yz_passes(pm, T, force_mesh, nullptr, nullptr, nullptr));
     if (force) HYMD_TRY(readout_sorted(pm, 3, T, force_mesh, force, false));
     return HYMD_OK;
 }
@@ -2017,20 +1442,21 @@ int hymd::update_field_force_q_impl(hymd_pm *pm, const float *x, const float *ch
     KGeom g = kgeom(pm);
     double *partials = energy_q ? (double *)pm->partials.ptr : nullptr;
     int nparts = pm->kblocks;
-    const XlineShape sh = xline_grad_shape(pm->fft, 1, pm->xline_w);
+    const XlineShape sh = xline_shape(pm->fft, 1, pm->xline_w, true);
+    HYMD_TRY(fft_r2c_zy(pm->fft, rho, spec, 1, s));
     if (sh.W > 0) {
-        // z + y forward passes, then one x-line pass: the forward x
-        // transform, the k-space pass and the inverse x transforms of
-        // -i k_x psi and psi
-        HYMD_TRY(fft_r2c_zy(pm->fft, rho, spec, 1, s));
-        FieldK fk{};
-        fk.T = 1;
-        HYMD_TRY(launch_xline_grad(pm, spec, out, g, fk, sh, partials, &nparts, &p));
+        XlineJob job;
+        job.spec = spec;
+        job.out = out;
+        job.g = g;
+        job.pme = true;
+        job.pk = p;
+        job.partials = partials;
+        HYMD_TRY(xline_pass(pm->fft, sh, job, &nparts, s));
     } else {
-        HYMD_TRY(fft_r2c_real(pm->fft, rho, spec, 1, s));
-        pme_kspace_kernel<<<pm->kblocks, kBlock, 0, s>>>(spec, out, psi ? 1 : 0, 1, g, p, partials);
+        HYMD_TRY(fft_forward_x(pm->fft, spec, 1, s));
+        pme_kspace_kernel<<<pm->kblocks, kBlock, 0, s>>>(spec, out, g, p, partials);
         HYMD_HIP(hipGetLastError());
-        // x-inverse of -i k_x psi and psi
         HYMD_TRY(fft_inverse_x(pm->fft, out, 2, s));
     }
     float *field = elec_field;
@@ -2038,15 +1464,8 @@ int hymd::update_field_force_q_impl(hymd_pm *pm, const float *x, const float *ch
         HYMD_TRY(pm->rscratch.reserve(sizeof(float) * 3 * m.g));
         field = (float *)pm->rscratch.ptr;
     }
-    // the plane pass (or the y and z line passes) forms E_y, E_z from psi
-    if (pm->fft.lds_plane) {
-        HYMD_TRY(fft_c2r_yz_grad(pm->fft, out, field, 1, g.kfac[1], g.kfac[2], 1.f, s));
-    } else {
-        HYMD_TRY(pm->cscratch.reserve(sizeof(float2) * m.gc * 3));
-        HYMD_TRY(fft_c2r_lines_grad(pm->fft, out, (float2 *)pm->cscratch.ptr, field, 1, g.kfac[1], g.kfac[2], 1.f,
-                                    s));
-    }
-    if (psi) HYMD_TRY(fft_c2r_yz(pm->fft, out + m.gc, psi, 1, 1.f, s));
+    // the y-z pass forms E_y, E_z and psi from psi's x-inverse spectrum
+    HYMD_TRY(yz_passes(pm, 1, field, psi, nullptr, nullptr));
     HYMD_TRY(readout_sorted(pm, 3, 1, field, elec_forces, true, accumulate));
     if (energy_q) {
         double e = 0.0;

@@ -142,6 +142,74 @@ __device__ __forceinline__ void kvec(const KGeom &g, int64_t kk64, double k[3], 
     wgt = (iz == 0 || 2 * iz == g.mz) ? 1.0 : 2.0;
 }
 
+// Quadratic form and filter of the field's k-space pass.
+struct FieldK {
+    int T;
+    int want_energy;
+    double sigma2;   // sigma^2
+    double inv_g;    // 1/G (r2c normalisation)
+    double c0;
+    double Ad[HYMD_MAX_TYPES * HYMD_MAX_TYPES];
+    double b[HYMD_MAX_TYPES];
+    float Af[HYMD_MAX_TYPES * HYMD_MAX_TYPES];
+};
+
+struct PmeK {
+    double sigma2;
+    double inv_g;
+    double four_pi_elec;  // 4 pi k_e / eps_r
+};
+
+// The quadratic Hamiltonian's k-space pass at element kk.  spec[t] = unnormalised
+// FFT of rho_t = paint_t/dV; out[t] = -i k_x V_t and out[T + t] = V_t (what the
+// inverse x transforms take), phif[t] = H rho_t/G (optional).  Returns the
+// element's energy (0 unless p.want_energy).
+template <int MAXT>
+__device__ __forceinline__ double kspace_point(const float2 *__restrict__ spec, float2 *__restrict__ out,
+                                               float2 *__restrict__ phif, const KGeom &g, const FieldK &p,
+                                               int64_t kk) {
+    double k[3], kd[3], wgt;
+    kvec(g, kk, k, kd, wgt);
+    const double k2 = k[0] * k[0] + k[1] * k[1] + k[2] * k[2];
+    const float H = (float)exp(-0.5 * p.sigma2 * k2);
+    const float hn = (float)((double)H * p.inv_g);
+    float2 ph[MAXT];
+#pragma unroll
+    for (int t = 0; t < MAXT; ++t) ph[t] = t < p.T ? cscale(spec[(int64_t)t * g.gc + kk], hn) : make_float2(0.f, 0.f);
+    if (phif) {
+#pragma unroll
+        for (int t = 0; t < MAXT; ++t)
+            if (t < p.T) phif[(int64_t)t * g.gc + kk] = ph[t];
+    }
+    const float kx = (float)kd[0];
+    double en = 0.0;
+#pragma unroll 1
+    for (int t = 0; t < p.T; ++t) {
+        float2 v = make_float2(0.f, 0.f), own = v;
+#pragma unroll
+        for (int s = 0; s < MAXT; ++s) {
+            const float a = p.Af[t * HYMD_MAX_TYPES + s];  // zero beyond T
+            v.x += a * ph[s].x;
+            v.y += a * ph[s].y;
+            if (s == t) own = ph[s];
+        }
+        if (p.want_energy) {
+            double e = 0.0;
+#pragma unroll
+            for (int s = 0; s < MAXT; ++s)
+                e += p.Ad[t * HYMD_MAX_TYPES + s] * ((double)own.x * (double)ph[s].x + (double)own.y * (double)ph[s].y);
+            en += 0.5 * wgt * e;
+            if (kk == 0) en += p.b[t] * (double)own.x;
+        }
+        v = cscale(v, H);
+        if (kk == 0) v.x += (float)p.b[t];
+        out[(int64_t)t * g.gc + kk] = make_float2(kx * v.y, -kx * v.x);
+        out[(int64_t)(p.T + t) * g.gc + kk] = v;
+    }
+    if (p.want_energy && kk == 0) en += p.c0;
+    return en;
+}
+
 // Moments kernel instance for T types (MAXT = 2, 4 or 8), its partial row
 // length 2 NP + MAXT, and its block count for a half spectrum of gc
 // elements (about 8 elements per thread).

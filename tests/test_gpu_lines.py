@@ -1,0 +1,77 @@
+"""The line transforms and the x-line pass at the sizes where their plans
+change: every radix of a stage, one- to four-stage lines, y-z planes of both
+register budgets and the separate line passes, and every number of types of
+the x-line pass (1 to 8, 9 beyond it, Mx = 4 without it)."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import field as F
+from tests.conftest import rms_rel
+
+pytestmark = pytest.mark.gpu
+
+
+def _dev(a, dtype):
+    return torch.as_tensor(np.ascontiguousarray(a)).to(dtype).cuda().contiguous()
+
+
+@pytest.mark.parametrize("mesh", [(4, 4, 4), (6, 10, 6), (18, 10, 10), (30, 12, 16), (50, 54, 18), (90, 150, 20),
+                                  (16, 162, 54), (8, 30, 250), (12, 90, 60), (24, 100, 100), (6, 144, 150),
+                                  (6, 150, 200), (4, 750, 8), (480, 4, 6), (900, 6, 4), (4, 8, 1024),
+                                  (4, 192, 192), (10, 240, 250)])
+def test_line_plans_vs_numpy(hip, mesh):
+    """r2c and c2r against numpy in FP64; an FP32 transform's error grows like
+    sqrt(log G) ulp: 2e-6 of the spectrum's RMS, 2e-5 of the largest value back."""
+    from hymd_amd.field import ParticleMesh
+    rng = np.random.default_rng(sum(mesh))
+    pm = ParticleMesh(mesh, (1.0, 1.0, 1.0), 2)
+    x = rng.normal(size=(2,) + mesh).astype(np.float32)
+    ref = np.fft.rfftn(x.astype(np.float64), axes=(1, 2, 3))
+    X = pm.r2c(_dev(x, torch.float32)).cpu().numpy()
+    assert np.sqrt(np.mean(np.abs(X - ref) ** 2)) / np.sqrt(np.mean(np.abs(ref) ** 2)) < 2e-6
+    y = pm.c2r(_dev(ref.astype(np.complex64), torch.complex64)).cpu().numpy()
+    np.testing.assert_allclose(y / np.prod(mesh), x, atol=2e-5 * np.abs(x).max())
+
+
+@pytest.mark.parametrize("mesh", [(4, 6, 8), (6, 4, 6), (18, 10, 12), (16, 30, 20), (30, 16, 10), (128, 8, 6),
+                                  (150, 6, 8), (96, 10, 16), (256, 6, 4), (64, 20, 18), (8, 100, 100), (4, 150, 160),
+                                  (6, 192, 200)])
+@pytest.mark.parametrize("T", [1, 2, 3, 4, 5, 6, 7, 8, 9])
+def test_field_pass_matches_oracle(hip, mesh, T):
+    """Force grids, densities, their spectra, potentials and energy of one
+    update against the FP64 oracle (1e-5 and 1e-6 of each one's RMS), and the
+    force grids of the update that returns nothing else."""
+    from hymd_amd.field import ParticleMesh
+    rng = np.random.default_rng(sum(mesh) + T)
+    box = np.array(mesh) * 0.25
+    n = 3000
+    x = (rng.uniform(0, 1, (n, 3)) * box).astype(np.float32)
+    types = rng.integers(0, T, n).astype(np.int32)
+    A = rng.uniform(0.0, 1.0, (T, T))
+    A = A + A.T + T * np.eye(T)
+    b = rng.uniform(-1, 1, T)
+    ham = F.Quadratic(A, b, 0.3)
+    ref = F.update_field(x.astype(np.float64), types, T, mesh, box, 0.4, ham, compute_potential=True)
+    pm = ParticleMesh(mesh, box, T)
+    xd, td = _dev(x, torch.float32), _dev(types, torch.int32)
+    only, fm = pm.create("real", batch=(T, 3)), pm.create("real", batch=(T, 3))
+    phi, v, phif = pm.create("real", batch=T), pm.create("real", batch=T), pm.create("complex", batch=T)
+    pm.field_update(xd, td, T, A, b, 0.3, [1.0] * T, 0.4, only)
+    e = pm.field_update(xd, td, T, A, b, 0.3, [1.0] * T, 0.4, fm, phi=phi, phi_fourier=phif, v_ext=v,
+                        want_energy=True)
+    want = np.array([[ref["force_mesh"][t][d] for d in range(3)] for t in range(T)])
+    assert rms_rel(only.cpu().numpy(), want) < 1e-5
+    assert rms_rel(fm.cpu().numpy(), want) < 1e-5
+    assert rms_rel(phi.cpu().numpy(), np.array(ref["phi"])) < 1e-6
+    assert rms_rel(v.cpu().numpy(), np.array(ref["v_ext"])) < 1e-6
+    assert rms_rel(phif.cpu().numpy(), np.array(ref["phi_fourier"])) < 1e-6
+    assert e == pytest.approx(F.field_energy(ref["phi"], ham, mesh, box), rel=1e-6)
+
+
+def test_edges_refused(hip):
+    from hymd_amd._lib import HymdError
+    from hymd_amd.field import ParticleMesh
+    for mesh in ((250, 8, 8), (8, 486, 8), (500, 8, 8), (8, 960, 8), (8, 14, 8)):
+        with pytest.raises(HymdError):
+            ParticleMesh(mesh, (1.0, 1.0, 1.0), 1)
