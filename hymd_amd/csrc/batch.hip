@@ -59,30 +59,43 @@ __device__ __forceinline__ int find_range(const int64_t *__restrict__ off, int R
 // (chunk_in[c] = (slot, end of its replica) of particle 64c, built with the
 // handle) gives it, and only the lanes past its end (a wavefront that
 // straddles two replicas) search on their own.
+// ITEMS: 1, or kRankItems of the workgroup ranked together.
+template <int ITEMS>
 __global__ void __launch_bounds__(kBlock) batch_key_kernel(const float *__restrict__ x, int64_t n,
                                                             const int64_t *__restrict__ poff, int R,
                                                             const int *__restrict__ slot_of,
                                                             const int2 *__restrict__ chunk_in,
                                                             const RepGeom *__restrict__ geo, int2 *__restrict__ keys,
                                                             int *__restrict__ counts) {
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t i0 = (int64_t)xcd_block(blockIdx.x, gridDim.x) * blockDim.x; i0 < n;
-         i0 += stride) {  // uniform per wavefront
-        const int64_t i = i0 + threadIdx.x;
-        const int wbase = __builtin_amdgcn_readfirstlane((int)(i0 + (threadIdx.x & ~63u)));
-        int key = -1;
+    const int64_t i0 = (int64_t)xcd_block(blockIdx.x, gridDim.x) * (ITEMS * kBlock) + threadIdx.x;
+    int key[ITEMS], rank[ITEMS];
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j) {
+        const int64_t i = i0 + j * kBlock;
+        const int64_t wbase = i - (threadIdx.x & 63);  // uniform per wavefront
+        key[j] = -1;
+        rank[j] = 0;
         if (wbase < n) {
-            const int2 ck = chunk_in[wbase >> 6];
+            const int2 ck = chunk_in[__builtin_amdgcn_readfirstlane((int)(wbase >> 6))];
             const RepGeom *G = geo + ck.x;
             if (i < n && i >= ck.y) G = geo + slot_of[find_range(poff, R, i)];
             if (i < n) {
                 const CicAxis cx = cic_axis((double)x[3 * i + 0], G->inv_h[0], G->mx);
                 const CicAxis cy = cic_axis((double)x[3 * i + 1], G->inv_h[1], G->my);
-                key = G->row_off + cx.i0 * G->my + cy.i0;
+                key[j] = G->row_off + cx.i0 * G->my + cy.i0;
             }
         }
-        const int rank = rank_in_bin_all(key, counts);
-        if (i < n) keys[i] = make_int2(key, rank);
+    }
+    if constexpr (ITEMS == 1) {
+        rank[0] = rank_in_bin_all(key[0], counts);
+    } else {
+        __shared__ RankTable tab;
+        rank_in_bin_block(key, rank, tab, counts);
+    }
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j) {
+        const int64_t i = i0 + j * kBlock;
+        if (i < n) keys[i] = make_int2(key[j], rank[j]);
     }
 }
 
@@ -315,12 +328,14 @@ static YzJob force_job(const hymd_batch *b, const RepGroup &gp) {
 static int batch_enqueue(hymd_batch *b, const float *x, const int32_t *types, float *forces) {
     hipStream_t s = b->stream;
     const int S = b->R;
-    if (b->n > 0)
-        batch_key_kernel<<<grid_for(b->n), kBlock, 0, s>>>(x, b->n, (const int64_t *)b->d_poff.ptr, b->R,
-                                                           (const int *)b->d_slot_of.ptr,
-                                                           (const int2 *)b->d_chunk_in.ptr,
-                                                           (const RepGeom *)b->d_geo.ptr, (int2 *)b->keys.ptr,
-                                                           (int *)b->counts.ptr);
+    if (b->n > 0) {
+        // up to 2^20 particles the larger number of workgroups counts more (as in the single-mesh path)
+        const bool many = b->n > 1 << 20;
+        auto *kernel = many ? &batch_key_kernel<kRankItems> : &batch_key_kernel<1>;
+        kernel<<<grid_for(b->n, many ? kRankItems * kBlock : kBlock, 1 << 23), kBlock, 0, s>>>(
+            x, b->n, (const int64_t *)b->d_poff.ptr, b->R, (const int *)b->d_slot_of.ptr,
+            (const int2 *)b->d_chunk_in.ptr, (const RepGeom *)b->d_geo.ptr, (int2 *)b->keys.ptr, (int *)b->counts.ptr);
+    }
     HYMD_HIP(hipGetLastError());
     HYMD_TRY(exclusive_scan((int *)b->counts.ptr, (int *)b->start.ptr, b->rows, (int *)b->tiles.ptr, nullptr,
                             true, s));

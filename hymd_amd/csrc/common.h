@@ -184,6 +184,73 @@ __device__ __forceinline__ int rank_in_bin_all(int key, int *counts) {
     return key >= 0 ? base + offset : 0;
 }
 
+// rank_in_bin for the kRankItems items of every thread of a workgroup, with one
+// global atomic per distinct bin of the workgroup where the input is
+// spatially ordered (some wavefront's first bin holds 8 items or more): the items are
+// counted per bin in an LDS hash table (open addressing, twice as many slots
+// as items, so a probe always ends), each used slot reserves its ranks, all
+// of them in flight together, and an item's rank is its slot's base plus its
+// count.  Each wavefront enters the items that share its first item's bin as
+// one, so they do not queue on one slot.  Ordered wavefronts of one mesh row
+// wait on the same counter: 16.8M positions on 256^2 rows took 407 us with
+// rank_in_bin_all, 220 us here, 2.1M on 128 x 120 rows 34 and 25 us.
+// Unordered items take rank_in_bin_all, which has no table to clear (351k on
+// 6480 rows: 14.7 us, 18.7 us through the table).  Every thread of the
+// workgroup must call it, once per table.
+constexpr int kRankItems = 4;
+constexpr int kRankSlots = 2 * kRankItems * kBlock;
+struct RankTable {
+    int key[kRankSlots], count[kRankSlots];
+};
+
+__device__ __forceinline__ void rank_in_bin_block(const int (&key)[kRankItems], int (&rank)[kRankItems],
+                                                  RankTable &tab, int *counts) {
+    const unsigned long long head = __ballot(key[0] >= 0);
+    const int head_key = __builtin_amdgcn_readlane(key[0], head ? __ffsll((long long)head) - 1 : 0);
+    if (!__syncthreads_or(__popcll(__ballot(key[0] == head_key) & head) >= 8)) {
+#pragma unroll
+        for (int j = 0; j < kRankItems; ++j) rank[j] = rank_in_bin_all(key[j], counts);
+        return;
+    }
+    for (int s = threadIdx.x; s < kRankSlots; s += kBlock) {
+        tab.key[s] = -1;
+        tab.count[s] = 0;
+    }
+    __syncthreads();
+    const int lane = threadIdx.x & 63;
+    int slot[kRankItems];
+#pragma unroll
+    for (int j = 0; j < kRankItems; ++j) {
+        slot[j] = -1;
+        const unsigned long long live = __ballot(key[j] >= 0);
+        if (live == 0) continue;  // uniform
+        const int first = __ffsll((long long)live) - 1;
+        const unsigned long long same = __ballot(key[j] == __builtin_amdgcn_readlane(key[j], first));
+        const bool shared = (same >> lane) & 1ull;
+        if (key[j] >= 0 && (!shared || lane == first)) {
+            unsigned s = ((unsigned)key[j] * 2654435761u) >> 16 & (kRankSlots - 1);
+            for (;;) {
+                const int old = atomicCAS(&tab.key[s], -1, key[j]);
+                if (old == -1 || old == key[j]) break;
+                s = (s + 1) & (kRankSlots - 1);
+            }
+            slot[j] = (int)s;
+            rank[j] = atomicAdd(&tab.count[s], shared ? __popcll(same) : 1);
+        }
+        const int s0 = __builtin_amdgcn_readlane(slot[j], first), r0 = __builtin_amdgcn_readlane(rank[j], first);
+        if (shared) {
+            slot[j] = s0;
+            rank[j] = r0 + __popcll(same & ((1ull << lane) - 1ull));
+        }
+    }
+    __syncthreads();
+    for (int s = threadIdx.x; s < kRankSlots; s += kBlock)
+        if (tab.count[s] > 0) tab.count[s] = atomicAdd(counts + tab.key[s], tab.count[s]);
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kRankItems; ++j) rank[j] = slot[j] >= 0 ? tab.count[slot[j]] + rank[j] : 0;
+}
+
 // Division by a divisor fixed at launch, as a multiply-high and a shift
 // (Granlund & Montgomery, "Division by invariant integers using
 // multiplication", PLDI 1994, round-up multiplier): with s = ceil(log2 d) and

@@ -106,6 +106,40 @@ __global__ void __launch_bounds__(kBlock) row_key_kernel(const float *__restrict
     }
 }
 
+// The same with kRankItems particles per thread (rank_in_bin_block).
+__global__ void __launch_bounds__(kBlock) row_key_block_kernel(const float *__restrict__ x, const float *__restrict__ w,
+                                                          int64_t n, Mesh m, int2 *__restrict__ keys,
+                                                          int *__restrict__ counts) {
+    __shared__ RankTable tab;
+    const int64_t i0 = (int64_t)xcd_block(blockIdx.x, gridDim.x) * (kRankItems * kBlock) + threadIdx.x;
+    int key[kRankItems], rank[kRankItems];
+#pragma unroll
+    for (int j = 0; j < kRankItems; ++j) {
+        const int64_t i = i0 + j * kBlock;
+        key[j] = -1;
+        rank[j] = 0;
+        if (i < n && !(w && w[i] == 0.f)) key[j] = base_row(x, i, m);
+    }
+    rank_in_bin_block(key, rank, tab, counts);
+#pragma unroll
+    for (int j = 0; j < kRankItems; ++j) {
+        const int64_t i = i0 + j * kBlock;
+        if (i < n) keys[i] = make_int2(key[j], rank[j]);
+    }
+}
+
+// Up to 2^20 particles the one-item kernel: there its four times as many
+// workgroups count more than the shared atomics.
+static int launch_row_keys(const float *x, const float *w, int64_t n, const Mesh &m, int2 *keys, int *counts,
+                           hipStream_t s) {
+    if (n > 1 << 20)
+        row_key_block_kernel<<<grid_for(n, kRankItems * kBlock, 1 << 22), kBlock, 0, s>>>(x, w, n, m, keys, counts);
+    else if (n > 0)
+        row_key_kernel<<<grid_for(n), kBlock, 0, s>>>(x, w, n, m, keys, counts);
+    HYMD_HIP(hipGetLastError());
+    return HYMD_OK;
+}
+
 __global__ void __launch_bounds__(kBlock) key_scatter_kernel(const float *__restrict__ x,
                                                               const int32_t *__restrict__ types,
                                                               const float *__restrict__ w, int64_t n,
@@ -870,8 +904,7 @@ static int sort_particles(hymd_pm *pm, const float *x, const int32_t *types, con
     HYMD_TRY(pm->xs.reserve(sizeof(float4) * nn));
     if (w) HYMD_TRY(pm->ws.reserve(sizeof(float) * nn));
     if (n > 0 && !keys_ready)
-        row_key_kernel<<<grid_for(n), kBlock, 0, s>>>(x, w, n, m, (int2 *)pm->keys.ptr, (int *)pm->counts.ptr);
-    HYMD_HIP(hipGetLastError());
+        HYMD_TRY(launch_row_keys(x, w, n, m, (int2 *)pm->keys.ptr, (int *)pm->counts.ptr, s));
     HYMD_TRY(exclusive_scan((int *)pm->counts.ptr, (int *)pm->start.ptr, nrows, (int *)pm->tiles.ptr, nullptr,
                             true, s));
     HYMD_TRY(launch_key_scatter(x, types, w, n, (const int2 *)pm->keys.ptr, (const int *)pm->start.ptr,
@@ -1179,8 +1212,7 @@ int row_order(hymd_pm *pm, const float *x, int64_t n, int *order, hipStream_t s)
     if (n == 0) return HYMD_OK;
     const Mesh &m = pm->mesh;
     HYMD_TRY(pm->keys.reserve(sizeof(int2) * (size_t)n));
-    row_key_kernel<<<grid_for(n), kBlock, 0, s>>>(x, nullptr, n, m, (int2 *)pm->keys.ptr, (int *)pm->counts.ptr);
-    HYMD_HIP(hipGetLastError());
+    HYMD_TRY(launch_row_keys(x, nullptr, n, m, (int2 *)pm->keys.ptr, (int *)pm->counts.ptr, s));
     HYMD_TRY(exclusive_scan((int *)pm->counts.ptr, (int *)pm->start.ptr, (int64_t)m.mx * m.my, (int *)pm->tiles.ptr,
                             nullptr, true, s));
     row_order_kernel<<<grid_for(n), kBlock, 0, s>>>((const int2 *)pm->keys.ptr, n, (const int *)pm->start.ptr, order);

@@ -75,3 +75,27 @@ def test_edges_refused(hip):
     for mesh in ((250, 8, 8), (8, 486, 8), (500, 8, 8), (8, 960, 8), (8, 14, 8)):
         with pytest.raises(HymdError):
             ParticleMesh(mesh, (1.0, 1.0, 1.0), 1)
+
+
+# either side of the 2^20 particles from which the keys are ranked per
+# workgroup, with its shared table (ordered) and without (unordered)
+@pytest.mark.parametrize("n", [(1 << 20), (1 << 20) + 1, (1 << 20) + 1027])
+@pytest.mark.parametrize("ordered", [False, True])
+def test_binning_of_large_inputs(hip, n, ordered):
+    """Painted grids of the sorted path equal the scatter paint's bit for bit;
+    zero-weight particles and one crowded row among them."""
+    from hymd_amd.field import ParticleMesh
+    mesh, box, T = (18, 20, 16), (4.5, 5.0, 4.0), 2
+    rng = np.random.default_rng(n + ordered)
+    x = rng.uniform(0, 1, (n, 3)) * np.array(box)
+    x[: n // 8, :2] = 0.3
+    if ordered:
+        c = (x / 0.25).astype(np.int64)
+        x = x[np.lexsort((c[:, 2], c[:, 1], c[:, 0]))]
+    types = rng.integers(0, T, n).astype(np.int32)
+    pm = ParticleMesh(mesh, box, T)
+    xd, td = _dev(x, torch.float32), _dev(types, torch.int32)
+    grid = pm.paint_fixed(xd, td, T)
+    scat = torch.zeros((T,) + mesh, dtype=torch.int64, device="cuda")
+    pm.paint_fixed(xd, td, T, out=scat, accumulate=True)
+    assert torch.equal(grid.to(torch.int64), scat)
