@@ -99,3 +99,45 @@ def test_binning_of_large_inputs(hip, n, ordered):
     scat = torch.zeros((T,) + mesh, dtype=torch.int64, device="cuda")
     pm.paint_fixed(xd, td, T, out=scat, accumulate=True)
     assert torch.equal(grid.to(torch.int64), scat)
+
+
+# no iteration, one, several; a mesh whose x lines have no x-line pass (Mx = 4)
+@pytest.mark.parametrize("mesh,crit,conv", [((12, 10, 8), 2.0, "max_diff"), ((12, 10, 8), 0.99, "max_diff"),
+                                            ((12, 10, 8), 1e-7, "max_diff"), ((4, 12, 10), 1e-6, "max_diff"),
+                                            ((4, 12, 10), 1e-4, "csum"), ((30, 16, 18), 1e-9, "euclidean_norm")])
+def test_dielectric_iteration_counts(hip, mesh, crit, conv):
+    """The variable-dielectric loop, whose host looks at an iteration when the
+    next is enqueued: iterations (to within one, the criterion being met to
+    FP32 rounding), potential and polarisation (1e-4 and 1e-3 of their RMS)
+    against the FP64 oracle."""
+    from hymd_amd import config as C
+    from hymd_amd import field as HF
+    from oracle import gpe as OG
+    rng = np.random.default_rng(3)
+    L, T, n = np.array(mesh) * 0.4, 2, 3000
+    x = (rng.uniform(0, 1, (n, 3)) * L).astype(np.float32)
+    types = (x[:, 2] > 0.5 * L[2]).astype(np.int32)
+    q = np.zeros(n, dtype=np.float32)
+    q[:200], q[200:400] = 1.0, -1.0
+    cfg = C.Config(n_steps=1, time_step=0.03, mesh_size=mesh, sigma=0.6, kappa=0.05, box_size=L, n_types=T,
+                   coulombtype="PIC_Spectral_GPE", dielectric_type=[20.0, 80.0], type_charges=[0.5, -0.5],
+                   conv_crit=crit, convergence_type=conv)
+    pm, fields, elec, coul = HF.initialize_pm(None, cfg)
+    ref_phi = F.update_field(x.astype(np.float64), types, T, mesh, L, cfg.sigma,
+                             F.Quadratic(np.eye(T), np.zeros(T), 0.0))["phi"]
+    ph = _dev(np.array(ref_phi), torch.float32)
+    phi_q, phi_q_f, psi, efield = elec
+    eps, eps_f, eta, eta_f, pol, pol_prev, _, contrib, vbar, vbar_f, fme, fme_f = coul
+    forces = torch.empty((n, 3), dtype=torch.float32, device="cuda")
+    HF.update_field_force_q_GPE(None, [ph[t] for t in range(T)], _dev(types, torch.int32), _dev(q, torch.float32),
+                                phi_q, phi_q_f, eps, eps_f, eta, eta_f, pol_prev, pol, efield, forces, contrib, psi,
+                                vbar, vbar_f, fme, fme_f, None, None, None, pm, _dev(x, torch.float32), cfg)
+    ref = OG.update_field_force_q_gpe(x.astype(np.float64), types, q.astype(np.float64), ref_phi, mesh, L, cfg.sigma,
+                                      cfg.dielectric_type, cfg.type_charges, cfg.coulomb_constant,
+                                      conv_crit=cfg.conv_crit, conv=conv, phi_eps=np.zeros(mesh),
+                                      elec_field_contrib=np.zeros(mesh))
+    assert abs(pm.gpe_iterations - ref["iterations"]) <= (1 if crit < 0.5 else 0)
+    assert rms_rel(psi.cpu().numpy(), ref["psi"]) < 1e-4
+    if ref["iterations"]:
+        assert rms_rel(pol.cpu().numpy(), ref["phi_pol"]) < 1e-3
+    assert rms_rel(forces.cpu().numpy(), ref["forces"]) < 1e-4
