@@ -141,3 +141,34 @@ def test_dielectric_iteration_counts(hip, mesh, crit, conv):
     if ref["iterations"]:
         assert rms_rel(pol.cpu().numpy(), ref["phi_pol"]) < 1e-3
     assert rms_rel(forces.cpu().numpy(), ref["forces"]) < 1e-4
+
+
+@pytest.mark.parametrize("bad", [-1, 40])
+@pytest.mark.parametrize("energies", [False, True])
+def test_bonded_index_out_of_range(hip, bad, energies):
+    """The stateless kernels find a bad index while the forces are enqueued:
+    the call is refused, the forces stay as they were, the next call works."""
+    import ctypes
+    from hymd_amd import _lib
+    n, m = 40, 39
+    x = torch.rand((n, 3), device="cuda", dtype=torch.float32)
+    a = torch.arange(m, device="cuda", dtype=torch.int32)
+    b = a + 1
+    k, r0 = torch.ones(m, device="cuda", dtype=torch.float64), torch.full((m,), 0.1, device="cuda", dtype=torch.float64)
+    box = (ctypes.c_double * 3)(2.0, 2.0, 2.0)
+    e, pr = ctypes.c_double(-7.0), (ctypes.c_double * 3)()
+
+    def bonds(second, f):
+        _lib.call("hymd_cbf", f.data_ptr(), x.data_ptr(), n, box, a.data_ptr(), second.data_ptr(), r0.data_ptr(),
+                  k.data_ptr(), m, _lib.HYMD_F32, ctypes.byref(e) if energies else None,
+                  pr if energies else None, None)
+
+    f = torch.full((n, 3), 5.0, device="cuda", dtype=torch.float32)
+    wrong = b.clone()
+    wrong[7] = bad
+    torch.cuda.synchronize()
+    with pytest.raises(_lib.HymdError):
+        bonds(wrong, f)
+    assert e.value == -7.0 and bool((f == 5.0).all())
+    bonds(b, f)
+    assert not bool((f == 5.0).any())
