@@ -172,3 +172,27 @@ def test_bonded_index_out_of_range(hip, bad, energies):
     assert e.value == -7.0 and bool((f == 5.0).all())
     bonds(b, f)
     assert not bool((f == 5.0).any())
+
+
+@pytest.mark.parametrize("T", [1, 2, 3, 4, 5, 6, 7, 8])
+def test_force_adjoint_of_every_type_count(hip, T):
+    """dL/dA_ts of L = sum_i g_i . F_i is L at the unit coupling E_ts (the
+    forces are linear in A); FP64 oracle forces, 1e-5 of the largest entry (FP32 spectra)."""
+    from hymd_amd.autograd import field_adjoint
+    from hymd_amd.field import ParticleMesh
+    rng = np.random.default_rng(T)
+    mesh, box, n, sigma = (12, 10, 16), np.array((3.0, 2.5, 4.0)), 700, 0.5
+    x = (rng.uniform(0, 1, (n, 3)) * box).astype(np.float32)
+    types = rng.integers(0, T, n).astype(np.int32)
+    g = rng.normal(size=(n, 3)).astype(np.float32)
+    pm = ParticleMesh(mesh, box, T)
+    dA, _ = field_adjoint(pm, _dev(x, torch.float32), _dev(types, torch.int32), T, sigma, np.eye(T),
+                          _dev(g, torch.float32))
+    x64, ref = x.astype(np.float64), np.zeros((T, T))
+    for t in range(T):
+        for u in range(T):
+            E = np.zeros((T, T))
+            E[t, u] = 1.0
+            out = F.update_field(x64, types, T, mesh, box, sigma, F.Quadratic(E, np.zeros(T), 0.0))
+            ref[t, u] = np.sum(g * F.compute_field_force(x64, types, out["force_mesh"], mesh, box))
+    np.testing.assert_allclose(dA, ref, rtol=0, atol=1e-5 * np.abs(ref).max())
