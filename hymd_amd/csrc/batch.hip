@@ -254,12 +254,12 @@ __global__ void __launch_bounds__(kBlock) batch_readout_kernel(const float *__re
 }
 
 // grid (nb of the group, slots of the group)
-template <int MAXT>
+template <int T>
 __global__ void __launch_bounds__(kBlock) batch_moments_kernel(const float2 *__restrict__ spec,
-                                                                const RepGeom *__restrict__ geo, int slot0, int T,
+                                                                const RepGeom *__restrict__ geo, int slot0,
                                                                 const double *__restrict__ sigma2,
                                                                 double *__restrict__ partials) {
-    constexpr int ROW = 2 * (MAXT * (MAXT + 1) / 2) + MAXT;
+    constexpr int ROW = T * (T + 1) + T;
     const int slot = slot0 + (int)blockIdx.y;
     const RepGeom &G = geo[slot];
     KGeom g;
@@ -269,7 +269,7 @@ __global__ void __launch_bounds__(kBlock) batch_moments_kernel(const float2 *__r
     g.zh = G.zh;
     g.gc = G.gc;
     for (int d = 0; d < 3; ++d) g.kfac[d] = G.kfac[d];
-    moments_block<MAXT>(spec + G.spec_off, g, T, sigma2[slot], 1.0 / (double)G.g, blockIdx.x, gridDim.x,
+    moments_block<T>(spec + G.spec_off, g, sigma2[slot], 1.0 / (double)G.g, blockIdx.x, gridDim.x,
                         partials + (G.part_off + blockIdx.x) * ROW);
 }
 
@@ -352,21 +352,14 @@ static int batch_enqueue(hymd_batch *b, const float *x, const int32_t *types, fl
         HYMD_TRY(fft_r2c_real(gp->plan, (const float *)b->rho.ptr + G0.grid_off,
                               (float2 *)b->spec.ptr + G0.spec_off, gp->count * b->T, s));
         dim3 grid((unsigned)gp->nb, (unsigned)gp->count);
-        if (b->T <= 2)
-            batch_moments_kernel<2><<<grid, kBlock, 0, s>>>((const float2 *)b->spec.ptr,
-                                                            (const RepGeom *)b->d_geo.ptr, gp->first, b->T,
-                                                            (const double *)b->d_sigma2.ptr,
-                                                            (double *)b->partials.ptr);
-        else if (b->T <= 4)
-            batch_moments_kernel<4><<<grid, kBlock, 0, s>>>((const float2 *)b->spec.ptr,
-                                                            (const RepGeom *)b->d_geo.ptr, gp->first, b->T,
-                                                            (const double *)b->d_sigma2.ptr,
-                                                            (double *)b->partials.ptr);
-        else
-            batch_moments_kernel<8><<<grid, kBlock, 0, s>>>((const float2 *)b->spec.ptr,
-                                                            (const RepGeom *)b->d_geo.ptr, gp->first, b->T,
-                                                            (const double *)b->d_sigma2.ptr,
-                                                            (double *)b->partials.ptr);
+        using Kernel = void (*)(const float2 *, const RepGeom *, int, const double *, double *);
+        static constexpr Kernel by_types[8] = {batch_moments_kernel<1>, batch_moments_kernel<2>,
+                                               batch_moments_kernel<3>, batch_moments_kernel<4>,
+                                               batch_moments_kernel<5>, batch_moments_kernel<6>,
+                                               batch_moments_kernel<7>, batch_moments_kernel<8>};
+        by_types[b->T - 1]<<<grid, kBlock, 0, s>>>((const float2 *)b->spec.ptr, (const RepGeom *)b->d_geo.ptr,
+                                                   gp->first, (const double *)b->d_sigma2.ptr,
+                                                   (double *)b->partials.ptr);
         HYMD_HIP(hipGetLastError());
         if (forces) {
             dim3 kgrid((unsigned)std::min(grid_for(G0.gc), 1024), (unsigned)gp->count);

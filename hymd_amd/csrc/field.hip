@@ -429,12 +429,11 @@ __global__ void __launch_bounds__(kBlock) field_kspace_kernel(const float2 *__re
 
 // Spectral moments (P, Q, phi~(0)) of the filtered densities, one partial
 // row per block.
-template <int MAXT>
-__global__ void __launch_bounds__(kBlock) field_moments_kernel(const float2 *__restrict__ spec, KGeom g, int T,
+template <int T>
+__global__ void __launch_bounds__(kBlock) field_moments_kernel(const float2 *__restrict__ spec, KGeom g,
                                                                 double sigma2, double inv_g,
                                                                 double *__restrict__ partials) {
-    moments_block<MAXT>(spec, g, T, sigma2, inv_g, blockIdx.x, gridDim.x,
-                        partials + (int64_t)blockIdx.x * (2 * (MAXT * (MAXT + 1) / 2) + MAXT));
+    moments_block<T>(spec, g, sigma2, inv_g, blockIdx.x, gridDim.x, partials + (int64_t)blockIdx.x * (T * (T + 1) + T));
 }
 
 // ---------------------------------------------------------------------------
@@ -1289,15 +1288,11 @@ extern "C" int hymd_field_moments(hymd_pm *pm, const float *x, const int32_t *ty
     HYMD_TRY(part.reserve(sizeof(double) * (size_t)row * nb));
     HYMD_TRY(pm->result.reserve(sizeof(double) * row));
     HYMD_TRY(pm->host.reserve(sizeof(double) * row));
-    if (T <= 2)
-        field_moments_kernel<2><<<nb, kBlock, 0, s>>>(spec, g, T, sigma * sigma, 1.0 / (double)m.g,
-                                                      (double *)part.ptr);
-    else if (T <= 4)
-        field_moments_kernel<4><<<nb, kBlock, 0, s>>>(spec, g, T, sigma * sigma, 1.0 / (double)m.g,
-                                                      (double *)part.ptr);
-    else
-        field_moments_kernel<8><<<nb, kBlock, 0, s>>>(spec, g, T, sigma * sigma, 1.0 / (double)m.g,
-                                                      (double *)part.ptr);
+    using Kernel = void (*)(const float2 *, KGeom, double, double, double *);
+    static constexpr Kernel by_types[8] = {field_moments_kernel<1>, field_moments_kernel<2>, field_moments_kernel<3>,
+                                           field_moments_kernel<4>, field_moments_kernel<5>, field_moments_kernel<6>,
+                                           field_moments_kernel<7>, field_moments_kernel<8>};
+    by_types[T - 1]<<<nb, kBlock, 0, s>>>(spec, g, sigma * sigma, 1.0 / (double)m.g, (double *)part.ptr);
     HYMD_HIP(hipGetLastError());
     HYMD_TRY(reduce_partials((const double *)part.ptr, nb, row, (double *)pm->result.ptr, s));
     HYMD_HIP(hipMemcpyAsync(pm->host.ptr, pm->result.ptr, sizeof(double) * row, hipMemcpyDeviceToHost, s));

@@ -196,3 +196,22 @@ def test_force_adjoint_of_every_type_count(hip, T):
             out = F.update_field(x64, types, T, mesh, box, sigma, F.Quadratic(E, np.zeros(T), 0.0))
             ref[t, u] = np.sum(g * F.compute_field_force(x64, types, out["force_mesh"], mesh, box))
     np.testing.assert_allclose(dA, ref, rtol=0, atol=1e-5 * np.abs(ref).max())
+
+
+@pytest.mark.parametrize("T", [1, 2, 3, 4, 5, 6, 7, 8])
+def test_moments_of_every_type_count(hip, T):
+    """Energy of one Hamiltonian from the spectral moments and from the field
+    update (FP64 sums of FP32 spectra in another order: 1e-6)."""
+    from hymd_amd.autograd import moments
+    from hymd_amd.field import ParticleMesh
+    rng = np.random.default_rng(T)
+    mesh, box, n, sigma = (12, 10, 16), np.array((3.0, 2.5, 4.0)), 900, 0.5
+    xd = _dev(rng.uniform(0, 1, (n, 3)) * box, torch.float32)
+    td = _dev(rng.integers(0, T, n), torch.int32)
+    A = rng.uniform(0, 1, (T, T)) + 2 * np.eye(T)
+    A = A + A.T
+    pm = ParticleMesh(mesh, box, T)
+    e = pm.field_update(xd, td, T, A, np.zeros(T), 0.0, [1.0] * T, sigma, pm.create("real", batch=(T, 3)),
+                        want_energy=True)
+    P = np.asarray(moments(pm, xd, td, T, sigma)[0])
+    assert 0.5 * np.prod(box) * np.sum(A * P) == pytest.approx(e, rel=1e-6)
