@@ -251,27 +251,6 @@ __device__ __forceinline__ void rank_in_bin_block(const int (&key)[kRankItems], 
     for (int j = 0; j < kRankItems; ++j) rank[j] = slot[j] >= 0 ? tab.count[slot[j]] + rank[j] : 0;
 }
 
-// Division by a divisor fixed at launch, as a multiply-high and a shift
-// (Granlund & Montgomery, "Division by invariant integers using
-// multiplication", PLDI 1994, round-up multiplier): with s = ceil(log2 d) and
-// m = floor(2^32 (2^s - d) / d) + 1, n / d = (umulhi(n, m) + n) >> s for every
-// 0 <= n < 2^31 (the sum cannot overflow since umulhi(n, m) <= n).  The FFT
-// stages use it where an integer divide would cost ~20 instructions per lane.
-struct FastDiv {
-    uint32_t d, m, s;
-};
-
-inline FastDiv make_fastdiv(uint32_t d) {
-    uint32_t s = 0;
-    while ((1ull << s) < d) ++s;
-    const uint64_t m = (((1ull << s) - d) << 32) / d + 1;
-    return FastDiv{d, (uint32_t)m, s};
-}
-
-__device__ __forceinline__ int fdiv(int n, const FastDiv &f) {
-    return (int)((__umulhi((uint32_t)n, f.m) + (uint32_t)n) >> f.s);
-}
-
 // mesh geometry passed by value to kernels
 struct Mesh {
     int mx, my, mz, zh;     // real edges, zh = mz/2+1

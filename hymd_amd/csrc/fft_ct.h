@@ -1,5 +1,5 @@
 // Line transforms whose length, line count and strides are known at compile
-// time, on radices 8, 4, 3, 5 in a fixed order: every index map is a shift or a
+// time, on radices 8, 4, 2, 5 in a fixed order: every index map is a shift or a
 // multiply-shift, the strides fold into the LDS offsets and a thread holds only
 // the butterflies it owns.
 //
@@ -27,17 +27,6 @@ __device__ __forceinline__ void small_dft<2>(float2 (&u)[8], float) {
     float2 a = u[0], b = u[1];
     u[0] = cadd(a, b);
     u[1] = csub(a, b);
-}
-
-template <>
-__device__ __forceinline__ void small_dft<3>(float2 (&u)[8], float sgn) {
-    const float h = 0.86602540378443864676f;  // sqrt(3)/2
-    float2 t = cadd(u[1], u[2]);
-    float2 m = make_float2(u[0].x - 0.5f * t.x, u[0].y - 0.5f * t.y);
-    float2 s = cmul_i(csub(u[1], u[2]), sgn * h);
-    u[0] = cadd(u[0], t);
-    u[1] = cadd(m, s);
-    u[2] = csub(m, s);
 }
 
 template <>
@@ -96,7 +85,7 @@ struct StagePlan {
 };
 
 // radices largest first: 8s, then one 4 / 4+4 / 2 for the power-of-two
-// remainder, then 3s and 5s (ns = 0 if n is not 2^a 3^b 5^c)
+// remainder, then 5s (ns = 0 if n is not 2^a 5^c)
 constexpr StagePlan make_stage_plan(int n) {
     StagePlan sp{};
     int rs[kMaxStages] = {};
@@ -119,10 +108,6 @@ constexpr StagePlan make_stage_plan(int n) {
     }
     for (int i = 0; i < eights; ++i) rs[cnt++] = 8;
     for (int i = 0; i < nt; ++i) rs[cnt++] = tail[i];
-    while (n % 3 == 0) {
-        n /= 3;
-        rs[cnt++] = 3;
-    }
     while (n % 5 == 0) {
         n /= 5;
         rs[cnt++] = 5;
