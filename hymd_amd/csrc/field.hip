@@ -1142,12 +1142,9 @@ static int kspace_pass(hymd_pm *pm, const FieldK &p, bool transformed, float2 *p
     job.g = kgeom(pm);
     job.p = p;
     job.partials = partials;
-    const XlineShape sh = xline_shape(pm->fft, T, pm->xline_w, !phif && !phix && !transformed);
-    // 4 T half spectra written in runs of 32 bytes: from 256 x points on they
-    // cost more than the separate passes (256^3, six types, with densities and
-    // spectra 4333 against 3022 us; 200^3 1533 against 1587, 144^3, eight types
-    // 797 against 768; 8 lines, 256^3, four types 1900 against 2045)
-    const bool narrow = (phif || phix) && sh.W < 8 && m.mx >= 256;
+    const bool more = phif || phix || transformed;
+    const XlineShape sh = xline_shape(pm->fft, T, pm->xline_w, !more);
+    const bool narrow = sh.W != pm->xline_w && xline_narrow(m, T, sh.W, more);  // a width asked for is taken
     if (sh.W > 0 && fused && !narrow) return xline_pass(pm->fft, sh, job, nblocks, s);
     if (!transformed) HYMD_TRY(fft_forward_x(pm->fft, (float2 *)pm->spec.ptr, T, s));
     if (phix && !phif) phif = phix;

@@ -39,14 +39,37 @@ XlineShape xline_shape(const FftPlan &plan, int T, int want, bool fixed);
 
 // Lines per workgroup of the pass on fft_ct.h, 0 where there is none: x edges
 // of 128 and 160 with up to four types, and 256 with one or with five and
-// more, whose 4 lines of the general pass (32-byte runs at a power-of-two
-// stride) cost more: 256^3, forces of 5, 7 and 8 types 2586, 3587 and 4934 us
-// there, 1726, 2391 and 2955 here.
+// more, where the general pass has 2 lines (16-byte runs): 256^3, forces of 5,
+// 7 and 8 types 2586, 3587 and 4934 us there, 1726, 2391 and 2955 here.
 inline int xline_fixed_lines(int n, int T, int want) {
     if (n == 128 && T <= 4) return T <= 2 ? 16 : 8;
     if (n == 160 && T <= 4) return T <= 2 ? 8 : 4;
     if (n == 256 && T == 1) return 8;
     return n == 256 && T >= 5 && T <= 8 ? (want == 4 && T == 6 ? 4 : 8) : 0;
+}
+
+// Whether W lines per workgroup (runs of 8 W bytes) are too few for the pass,
+// so that the separate passes (16 lines each) are the faster ones.  more: the
+// job also writes spectra and densities, or starts from held spectra; else it
+// makes the force grids only.  The whole call with the pass / separate, us:
+//   W = 1: 216^3, T = 8 2316 / 2093; 240^3, T = 8 2978 / 2643; up to two types
+//     keep it: 900 x 96 x 96, T = 1 251 / 263.
+//   W = 2: T = 8, 144^3 639 / 580, 160^3 687 / 645, 200^3 1539 / 1560; fewer
+//     types keep it: T = 6, 216^3 1460 / 1608, 240^3 1819 / 2002.
+//   Rows of 129 elements in multiples of 64, where the x stride is 2^k 129
+//   elements and the pass moves 0.8 to 1.6 TB/s against 1.7 to 2.0 on every other
+//   plane measured (64 to 256 rows of 33 to 161 elements; the strides seem to
+//   meet on few memory channels):
+//     W = 2: T = 6, 192 x 256 x 256 2305 / 1735, 240 x 256 x 256 2668 / 2228.
+//     W = 4: T = 4, 192 x 256 x 256 1123 / 1175; T = 6, 100 x 256 x 256 908 / 938,
+//       but where the types lie 2^k 129 elements apart as well T = 8, 128 x 256 x
+//       256 2000 / 1563, T = 6, 96 x 256 x 256 951 / 896.
+//     more: held spectra, W = 2, 256^3, T = 6 2488 / 1653; W = 4, 192 x 256 x 256,
+//       T = 4 874 / 825; densities, 288 x 256 x 256, T = 4 2429 / 2306.
+inline bool xline_narrow(const Mesh &m, int T, int W, bool more) {
+    const bool few_channels = m.zh == 129 && m.my % 64 == 0;
+    const int least = more || (T >= 6 && m.mx % 32 == 0) ? 4 : 2;
+    return (W == 1 && T >= 3) || (W == 2 && T >= 8) || (few_channels && W <= least);
 }
 
 struct XlineJob {

@@ -2,6 +2,8 @@
 change: every radix of a stage, one- to four-stage lines, y-z planes of both
 register budgets and the separate line passes, and every number of types of
 the x-line pass (1 to 8, 9 beyond it, Mx = 4 without it)."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -215,3 +217,50 @@ def test_moments_of_every_type_count(hip, T):
                         want_energy=True)
     P = np.asarray(moments(pm, xd, td, T, sigma)[0])
     assert 0.5 * np.prod(box) * np.sum(A * P) == pytest.approx(e, rel=1e-6)
+
+
+def _moment_grids(pm, xd, td, T, A, b, sigma):
+    """Force grids of the separate passes (hymd_field_moments), whose density
+    spectra the handle then holds; (grids, moments P, phi~(0))."""
+    from hymd_amd._lib import call, darr, dptr
+    grids = pm.create("real", batch=(T, 3))
+    nv = T * (T + 1) + T
+    out = (ctypes.c_double * nv)()
+    call("hymd_field_moments", pm.handle, dptr(xd, torch.float32), dptr(td, torch.int32), int(xd.shape[0]), T,
+         darr([1.0] * T), sigma, out, darr(np.ravel(A)), darr(b), dptr(grids, torch.float32))
+    m = np.array(out)
+    P = np.zeros((T, T))
+    P[np.triu_indices(T)] = m[: T * (T + 1) // 2]
+    return grids, P + np.triu(P, 1).T, m[T * (T + 1):]
+
+
+# one line per workgroup, two of eight types, two and four where the rows have
+# 129 elements: the separate passes; three shapes of the fused pass for contrast
+@pytest.mark.parametrize("mesh,T,separate", [((216, 12, 10), 8, True), ((240, 10, 8), 7, True),
+                                             ((144, 12, 10), 8, True), ((192, 64, 256), 6, True),
+                                             ((240, 64, 256), 4, True), ((240, 10, 8), 6, False),
+                                             ((192, 60, 256), 6, False), ((144, 12, 10), 7, False)])
+def test_held_spectra_route(hip, mesh, T, separate):
+    """Force grids from held spectra: where the x-line pass would run too few
+    lines per workgroup they come from the separate passes, bit for bit the
+    moments' own grids; else from the fused pass, equal to FP32 rounding (1e-6
+    of the RMS).  Both agree with the FP64 oracle."""
+    from hymd_amd._lib import call, darr, dptr
+    from hymd_amd.field import ParticleMesh
+    rng = np.random.default_rng(sum(mesh) + T)
+    box = np.array(mesh) * 0.25
+    n, sigma = 3000, 0.4
+    x = (rng.uniform(0, 1, (n, 3)) * box).astype(np.float32)
+    types = rng.integers(0, T, n).astype(np.int32)
+    A = rng.uniform(0.0, 1.0, (T, T))
+    A = A + A.T + T * np.eye(T)
+    b = rng.uniform(-1, 1, T)
+    pm = ParticleMesh(mesh, box, T)
+    grids, _, _ = _moment_grids(pm, _dev(x, torch.float32), _dev(types, torch.int32), T, A, b, sigma)
+    held = pm.create("real", batch=(T, 3))
+    call("hymd_field_forces_held", pm.handle, T, darr(np.ravel(A)), darr(b), sigma, dptr(held, torch.float32), None)
+    assert torch.equal(held, grids) == separate
+    assert rms_rel(held.cpu().numpy(), grids.cpu().numpy()) < 1e-6
+    ref = F.update_field(x.astype(np.float64), types, T, mesh, box, sigma, F.Quadratic(A, b, 0.0))
+    want = np.array([[ref["force_mesh"][t][d] for d in range(3)] for t in range(T)])
+    assert rms_rel(held.cpu().numpy(), want) < 1e-5
