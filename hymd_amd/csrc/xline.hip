@@ -10,7 +10,9 @@ namespace hymd {
 // narrower ones give the chip more blocks, so: 16 lines, halved while they
 // exceed the threads, half of a CU's LDS or a middle stage's registers, or
 // while the blocks would not fill the chip twice and the runs are longer than
-// 32 bytes.
+// 32 bytes.  Eight types fill a block's threads by themselves, so there once
+// is enough (update of 64^3, 264 blocks of 8 lines 98 us, 528 of 4 103; seven
+// types 92 and 88).
 XlineShape xline_shape(const FftPlan &plan, int T, int want, bool fixed) {
     XlineShape sh;
     const int n = plan.mesh.mx, lines = plan.mesh.my * plan.mesh.zh;
@@ -39,7 +41,7 @@ XlineShape xline_shape(const FftPlan &plan, int T, int want, bool fixed) {
             if (threads(W) <= 256 && fits(W, 40 * 1024)) sh.W = W;
         for (int W = 16; W >= 2 && !sh.W; W >>= 1)
             if (fits(W, 80 * 1024)) sh.W = W;
-        while (sh.W > 4 && lines / sh.W < 512 && fits(sh.W / 2, 80 * 1024)) sh.W /= 2;
+        while (sh.W > 4 && lines / sh.W < (T < 8 ? 512 : 256) && fits(sh.W / 2, 80 * 1024)) sh.W /= 2;
         for (int W = 2; W >= 1 && !sh.W; W >>= 1)
             if (fits(W, kXlineLdsBytes)) sh.W = W;
     }
