@@ -57,14 +57,17 @@ static LineRadices xline_radices(int n, int cap) {
     return LineRadices{};
 }
 
-// Whether every stage run in place on nlines lines fits `threads` threads of
-// at most `elems` values.
-static bool line_fits(const LineAxis &ax, int nlines, int threads, int elems) {
-    for (int s = 0; s < ax.ns; ++s)
+// Whether the stages [first, last) run in place on nlines lines fit `threads`
+// threads of at most `elems` values.
+static bool stages_fit(const LineAxis &ax, int nlines, int threads, int elems, int first, int last) {
+    for (int s = first; s < last; ++s)
         if ((int64_t)nlines * ax.st[s].nr > (int64_t)threads * std::max(1, elems / ax.st[s].R)) return false;
     return true;
 }
 
+static bool line_fits(const LineAxis &ax, int nlines, int threads, int elems) {
+    return stages_fit(ax, nlines, threads, elems, 0, ax.ns);
+}
 
 // Lines per workgroup of a strided pass: 16 (128 contiguous bytes per element
 // row), fewer where the middle stages or LDS do not take them.
@@ -78,6 +81,15 @@ static int strided_width(const LineAxis &ax) {
 
 static bool plane_fits(const FftPlan &plan, int threads, int elems) {
     return line_fits(plan.ly, plan.mesh.zh, threads, elems) && line_fits(plan.lzh, plan.mesh.my, threads, elems);
+}
+
+// The same for one direction: its first axis' first stage and its second axis'
+// last one do not run in place (an axis of one stage runs that one).
+static bool plane_fits(const FftPlan &plan, int threads, int elems, bool inverse) {
+    const LineAxis &a = inverse ? plan.ly : plan.lzh, &b = inverse ? plan.lzh : plan.ly;
+    const int na = inverse ? plan.mesh.zh : plan.mesh.my, nb = inverse ? plan.mesh.my : plan.mesh.zh;
+    return stages_fit(a, na, threads, elems, 1, a.ns) &&
+           stages_fit(b, nb, threads, elems, 0, std::max(1, b.ns - 1));
 }
 
 // Whether the y-z planes have a kernel compiled for their size (with_plane).
@@ -281,7 +293,7 @@ struct PlaneTables {
 // Any mesh: sizes, plans and strides known at launch.
 template <int ELEMS>
 struct PlaneRt {
-    static constexpr int threads = 1024, waves = 1;
+    static constexpr int threads = 1024, waves = ELEMS <= 16 ? 6 : 4;  // 80 and 128 registers
     int mx, my, nh, zh, zhs;
     float inv_my, inv_zh;
     LineAxis ay, az;
@@ -648,30 +660,42 @@ static size_t z_lds(const FftPlan &plan) {
     return sizeof(float2) * ((size_t)plan.lzh.n + plan.mesh.zh + (size_t)plan.wz * plan.zhs);
 }
 
-// Threads per workgroup of a plane kernel.  LDS lets k planes share a CU and
-// the registers 24 waves (16 with the larger register block), so a block gets
-// up to 24 / k of them; a launch of at most two planes per CU is bound by the
-// plane's own latency and takes up to 16.  Among those the count with the
-// fewest rounds of butterflies, weighted with their radix, then the smallest.
-static PlaneShape plane_shape(const FftPlan &plan, int64_t planes) {
-    const int k = planes <= 2 * kCus ? 1 : std::max(1, (int)(160 * 1024 / plan.lds_plane));
-    const int elems = plane_fits(plan, 1024, kLineElems) ? kLineElems : kPlaneElemsBig;
-    const int most = std::min(16, std::max(4, (elems == kLineElems ? 24 : 16) / k));
+// Threads and register block of a plane kernel: the fewest turns, times the
+// rounds of butterflies in a turn weighted with their radix.  Turns are the
+// planes over those the chip works on at a time, half way to whole; a CU holds
+// as many planes as LDS takes and as its SIMDs have registers for: PlaneRt::waves each, of which a workgroup takes a
+// quarter of its wavefronts, rounded up (so whole quarters are tried; and five
+// wavefronts of the smaller block, of which four workgroups were seen to fit).
+// A turn also costs about 35 rounds of radix 1 of its own: loads, stores,
+// barriers.  Gradient grids (c2r), the choice against the best of the others
+// tried (4 to 16 wavefronts of both blocks): 100^3, four types 28.0 / 33 us,
+// 96 x 200 x 96 61 / 69, 128 x 120 x 144, six types 103 / 118.  A rule that
+// counted 24 wavefronts per CU however they fall on the SIMDs took 13 of the
+// smaller block for planes of 75 to 81 KB, one plane per CU: 72 and 119 us in
+// the last two, and 17.8 us, now 13.9, for r2c of four grids of 100^3.
+static PlaneShape plane_shape(const FftPlan &plan, int64_t planes, bool inverse) {
+    const int in_lds = (int)(160 * 1024 / plan.lds_plane);
     PlaneShape best;
-    int best_cost = 1 << 30;
-    for (int w = 1; w <= 16; ++w) {
-        if (!plane_fits(plan, 64 * w, elems) || (w > most && best.threads)) continue;
-        int cost = 0;
-        for (const LineAxis *ax : {&plan.ly, &plan.lzh})
-            for (int s = 0; s < ax->ns; ++s) {
-                const int lines = ax == &plan.ly ? plan.mesh.zh : plan.mesh.my;
-                cost += (lines * ax->st[s].nr + 64 * w - 1) / (64 * w) * ax->st[s].R;
+    double best_cost = 0.0;
+    for (int w : {1, 2, 3, 4, 5, 8, 12, 16})
+        for (int elems : {kLineElems, kPlaneElemsBig}) {
+            const bool small = elems == kLineElems;
+            const int waves = small ? PlaneRt<kLineElems>::waves : PlaneRt<kPlaneElemsBig>::waves;
+            const int k = std::min(in_lds, w == 5 && small ? 4 : waves / ((w + 3) / 4));
+            if (k < 1 || !plane_fits(plan, 64 * w, elems, inverse)) continue;
+            int rounds = 35;
+            for (const LineAxis *ax : {&plan.ly, &plan.lzh})
+                for (int s = 0; s < ax->ns; ++s) {
+                    const int lines = ax == &plan.ly ? plan.mesh.zh : plan.mesh.my;
+                    rounds += (lines * ax->st[s].nr + 64 * w - 1) / (64 * w) * ax->st[s].R;
+                }
+            const double turns = (double)planes / (kCus * k), whole = std::ceil(turns);
+            const double cost = rounds * (turns < 1.0 ? 1.0 : 0.5 * (turns + whole));
+            if (!best.threads || cost < best_cost) {
+                best = PlaneShape{64 * w, elems};
+                best_cost = cost;
             }
-        if (cost < best_cost) {
-            best = PlaneShape{64 * w, elems};
-            best_cost = cost;
         }
-    }
     return best;
 }
 
@@ -687,12 +711,12 @@ static int lds_opt_in(K kernel, bool &done) {
 }
 
 // Calls f(geometry, threads) with the plane geometry for `planes` planes of
-// the plan: compile-time for the planes of the cubic meshes listed, whose
+// the plan in one direction: compile-time for the planes of the cubic meshes listed, whose
 // sizes the package's workloads use (128^2 on fft_ct.h, the four types of a
 // lipid/water step: c2r 48 us against 68 for the general form), else the
 // general one.
 template <class F>
-static int with_plane(const FftPlan &plan, int64_t planes, F &&f) {
+static int with_plane(const FftPlan &plan, int64_t planes, bool inverse, F &&f) {
     const Mesh &m = plan.mesh;
     const PlaneTables t{plan.ty, plan.tzh, plan.post}, tf{plan.fy, plan.fzh, plan.post};
     if (plane_fixed(m) && m.my == 128) return f(PlaneFixed<128, 128, 1024, 8>{m.mx, tf}, 1024);
@@ -704,7 +728,7 @@ static int with_plane(const FftPlan &plan, int64_t planes, F &&f) {
             default: return f(PlaneCt<96, 96, 512>{m.mx, t}, 512);
         }
     }
-    const PlaneShape sh = plane_shape(plan, planes);
+    const PlaneShape sh = plane_shape(plan, planes, inverse);
     const float iy = 1.0f / (float)m.my, iz = 1.0f / (float)m.zh;
     if (sh.elems == kLineElems)
         return f(PlaneRt<kLineElems>{m.mx, m.my, m.mz / 2, m.zh, plan.zhs, iy, iz, plan.ly, plan.lzh, t}, sh.threads);
@@ -774,7 +798,7 @@ int fft_r2c_zy(const FftPlan &plan, const float *in, float2 *out, int batch, hip
     const Mesh &m = plan.mesh;
     if (plan.lds_plane) {
         const int blocks = m.mx * batch;
-        return with_plane(plan, blocks, [&](auto g, int threads) -> int {
+        return with_plane(plan, blocks, false, [&](auto g, int threads) -> int {
             using G = decltype(g);
             static bool done = false;
             if (plan.lds_plane > 64 * 1024) HYMD_TRY(lds_opt_in(r2c_plane(g), done));
@@ -820,7 +844,7 @@ int fft_yz_multi(const FftPlan &plan, const YzJob &job, float2 *tmp, hipStream_t
     if (grids == 0) return HYMD_OK;
     if (plan.lds_plane) {
         const int blocks = plan.mesh.mx * grids;
-        return with_plane(plan, blocks, [&](auto g, int threads) -> int {
+        return with_plane(plan, blocks, true, [&](auto g, int threads) -> int {
             using G = decltype(g);
             static bool done = false;
             if (plan.lds_plane > 64 * 1024) HYMD_TRY(lds_opt_in(c2r_plane(g), done));

@@ -21,7 +21,11 @@ def _dev(a, dtype):
 @pytest.mark.parametrize("mesh", [(4, 4, 4), (6, 10, 6), (18, 10, 10), (30, 12, 16), (50, 54, 18), (90, 150, 20),
                                   (16, 162, 54), (8, 30, 250), (12, 90, 60), (24, 100, 100), (6, 144, 150),
                                   (6, 150, 200), (4, 750, 8), (480, 4, 6), (900, 6, 4), (4, 8, 1024),
-                                  (4, 192, 192), (10, 240, 250)])
+                                  (4, 192, 192), (10, 240, 250),
+                                  # several planes per CU (more than 256 of them): the register blocks and
+                                  # wavefronts chosen for planes of 2 KB to 150 KB
+                                  (150, 72, 256), (160, 200, 96), (150, 90, 72), (160, 54, 96), (270, 16, 18),
+                                  (160, 162, 108)])
 def test_line_plans_vs_numpy(hip, mesh):
     """r2c and c2r against numpy in FP64; an FP32 transform's error grows like
     sqrt(log G) ulp: 2e-6 of the spectrum's RMS, 2e-5 of the largest value back."""
