@@ -33,8 +33,9 @@ struct XlineShape {
     int W = 0, threads = 0, plan = 0;
     bool fixed = false;  // the pass of xline_fixed.hip
 };
-// want: lines wanted (0: any); fixed: the pass of xline_fixed.hip may be taken
-// (it makes the 2T inverse transforms and energies only).
+// want: lines wanted (0: any; others than the fixed pass has are the general
+// pass's, where they fit); fixed: the pass of xline_fixed.hip may be taken (it
+// makes the 2T inverse transforms and energies only).
 XlineShape xline_shape(const FftPlan &plan, int T, int want, bool fixed);
 
 // Lines per workgroup of the pass on fft_ct.h, 0 where there is none: x edges

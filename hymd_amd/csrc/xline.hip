@@ -17,12 +17,10 @@ XlineShape xline_shape(const FftPlan &plan, int T, int want, bool fixed) {
     XlineShape sh;
     const int n = plan.mesh.mx, lines = plan.mesh.my * plan.mesh.zh;
     if (T < 1 || T > 8) return sh;
-    sh.W = fixed ? xline_fixed_lines(n, T, want) : 0;
-    sh.fixed = sh.W > 0;
-    if (sh.fixed) return sh;
+    const int fixed_lines = fixed ? xline_fixed_lines(n, T, want) : 0;
     sh.plan = xline_plan_of(T);
     const LineAxis &ax = plan.xl[sh.plan].fwd;
-    if (ax.ns < 2) return sh;
+    if (ax.ns < 2) return sh;  // no fixed pass either
     const int nr2 = ax.st[ax.ns - 1].nr;
     auto threads = [&](int W) {
         const int t = std::max(W * nr2, std::min(256, T * W * ax.st[0].nr));
@@ -34,8 +32,12 @@ XlineShape xline_shape(const FftPlan &plan, int T, int want, bool fixed) {
             if (T * W * ax.st[s].nr > threads(W) * std::max(1, kXlineElems / ax.st[s].R)) return false;
         return true;
     };
-    if (want > 0 && fits(want, kXlineLdsBytes)) {
+    if (want > 0 && want != fixed_lines && fits(want, kXlineLdsBytes)) {
         sh.W = want;
+    } else if (fixed_lines > 0) {
+        sh.W = fixed_lines;
+        sh.fixed = true;
+        return sh;
     } else {
         for (int W = 16; W >= 8 && !sh.W; W >>= 1)
             if (threads(W) <= 256 && fits(W, 40 * 1024)) sh.W = W;

@@ -268,3 +268,39 @@ def test_held_spectra_route(hip, mesh, T, separate):
     ref = F.update_field(x.astype(np.float64), types, T, mesh, box, sigma, F.Quadratic(A, b, 0.0))
     want = np.array([[ref["force_mesh"][t][d] for d in range(3)] for t in range(T)])
     assert rms_rel(held.cpu().numpy(), want) < 1e-5
+
+
+# x edges with a fixed pass: 128, 160 and 256 points, a width that the general
+# pass takes there and the fixed pass's own
+@pytest.mark.parametrize("mesh,T,other,own", [((128, 20, 18), 2, 4, 16), ((128, 20, 18), 4, 4, 8),
+                                              ((160, 18, 20), 3, 2, 4), ((256, 12, 10), 5, 2, 8),
+                                              ((256, 12, 10), 6, 2, 8)])
+def test_xline_width_takes_effect(hip, mesh, T, other, own):
+    """The launch-shape knob: another width than the fixed x-line pass's runs
+    the general one, whose radices round differently (1e-6 of the RMS, not the
+    same bits), for the field update and for PME; the pass's own width and none
+    give the same bits."""
+    from hymd_amd import tune
+    from hymd_amd.field import ParticleMesh
+    rng = np.random.default_rng(sum(mesh) + T)
+    box = np.array(mesh) * 0.25
+    n = 3000
+    x = _dev(rng.uniform(0, 1, (n, 3)) * box, torch.float32)
+    types = _dev(rng.integers(0, T, n), torch.int32)
+    q = _dev(np.where(np.arange(n) % 2, 1.0, -1.0), torch.float32)
+    A = rng.uniform(0.0, 1.0, (T, T))
+    A = A + A.T
+    pm = ParticleMesh(mesh, box, T)
+
+    def grids(width):
+        tune.apply(pm, {"xline_width": width})
+        fm, ef = pm.create("real", batch=(T, 3)), pm.create("real", batch=3)
+        pm.field_update(x, types, T, A, np.zeros(T), 0.0, [1.0] * T, 0.4, fm)
+        pm.pme(x, q, 0.4, 1.0, 0.0, torch.empty_like(x), elec_field=ef)
+        return fm, ef
+
+    default, same, changed = grids(0), grids(own), grids(other)
+    assert torch.equal(same[0], default[0]) and not torch.equal(changed[0], default[0])
+    assert not torch.equal(changed[1], default[1])
+    for a, b in zip(changed, default):
+        assert rms_rel(a.cpu().numpy(), b.cpu().numpy()) < 1e-6
