@@ -198,8 +198,9 @@ __global__ void __launch_bounds__(G::threads, T * R2 <= 16 ? 4 : 1)
     // k_x of element e of the derivative (zero on the Nyquist plane)
     auto kdx = [&](int e) -> float { return 2 * e == n ? 0.f : (float)(g.kfac[0] * (2 * e < n ? e : e - n)); };
     double energy = 0.0;
+    float2 dx[PME ? R2 : 1];  // PME: -i k_x psi
     if constexpr (PME) {
-        // psi = 4 pi k_e / eps H rho / |k|^2 (|k|^2 := 1 at k = 0), in FP64
+        // psi = 4 pi k_e / eps H rho / |k|^2 (|k|^2 := 1 at k = 0) and -i k_x psi, in FP64
         if (active) {
 #pragma unroll
             for (int j = 0; j < R2; ++j) {
@@ -209,9 +210,10 @@ __global__ void __launch_bounds__(G::threads, T * R2 <= 16 ? 4 : 1)
                 if (line0 + l == 0 && e == 0) k2 = 1.0;
                 const double f = pk.four_pi_elec * (ex[e] * eyz) / k2;
                 const double rx = (double)u[0][j].x * pk.inv_g, ry = (double)u[0][j].y * pk.inv_g;
-                const double px = f * rx, py = f * ry;
+                const double px = f * rx, py = f * ry, kd = 2 * e == n ? 0.0 : kx;
                 if (l < wv) energy += 0.5 * wgt * (rx * px + ry * py);
                 u[0][j] = make_float2((float)px, (float)py);
+                dx[j] = make_float2((float)(kd * py), (float)(-kd * px));
             }
         }
     } else {
@@ -276,13 +278,14 @@ __global__ void __launch_bounds__(G::threads, T * R2 <= 16 ? 4 : 1)
             float kx[R2];
             const int fi = fresh(i);
 #pragma unroll
-            for (int j = 0; j < R2; ++j) kx[j] = f == 1 ? kdx(fi + j * nr2) : 0.f;
+            for (int j = 0; j < R2; ++j) kx[j] = !PME && f == 1 ? kdx(fi + j * nr2) : 0.f;
 #pragma unroll
             for (int t = 0; t < T; ++t) {
                 float2 c[R2];
 #pragma unroll
                 for (int j = 0; j < R2; ++j) {
-                    c[j] = f == 1 ? make_float2(kx[j] * u[t][j].y, -kx[j] * u[t][j].x) : u[t][j];
+                    if constexpr (PME) c[j] = f == 1 ? dx[j] : u[t][j];
+                    else c[j] = f == 1 ? make_float2(kx[j] * u[t][j].y, -kx[j] * u[t][j].x) : u[t][j];
                 }
                 dft::Dft<R2, 1>::run(c);
                 float2 *d = D + (t * W + l) * ld + i * R2;

@@ -304,3 +304,46 @@ def test_xline_width_takes_effect(hip, mesh, T, other, own):
     assert not torch.equal(changed[1], default[1])
     for a, b in zip(changed, default):
         assert rms_rel(a.cpu().numpy(), b.cpu().numpy()) < 1e-6
+
+
+@pytest.mark.parametrize("solver,axis", [("pme", 0), ("gpe", 0)])
+def test_derivative_factor_in_fp64(hip, solver, axis):
+    """The electric field of a charge density cos(2 k x) on eight points, whose
+    transforms are exact (factors of 1 and i), in a box whose k rounds to FP32
+    with a relative error of 5e-8 or more.  A field that multiplies by k in
+    FP64 is off by its roundings alone, which differ in sign over the 64
+    amplitudes (6e-8 at most each: 2e-8 bounds their mean); one that multiplies
+    by the rounded k is off by 5e-8 in every one."""
+    from hymd_amd._lib import call, darr, dptr
+    from hymd_amd.field import ParticleMesh
+    mesh = [8, 4, 4] if axis == 0 else [8, 8, 4] if axis == 1 else [8, 4, 8]
+    L = next(v for v in 3.0 + np.arange(320) / 64.0  # node positions are exact
+             if np.float32(2 * (2.0 * np.pi / v)) / (2 * (2.0 * np.pi / v)) - 1.0 > 5e-8)
+    k = 2 * (2.0 * np.pi / L)
+    box = np.full(3, 4.0)
+    box[axis] = L
+    pm = ParticleMesh(mesh, box, 1)
+    node = np.stack(np.meshgrid(*[np.arange(m) for m in mesh], indexing="ij"), -1).reshape(-1, 3)
+    x = _dev(node * (box / mesh), torch.float32)
+    wave = np.array([1.0, 0.0, -1.0, 0.0, 1.0, 0.0, -1.0, 0.0])[node[:, axis]]
+    odd = (node[:, axis] % 2 == 1).reshape(mesh)
+    dv = np.prod(box) / np.prod(mesh)
+    n = len(node)
+    errs = []
+    for s in np.linspace(1.0, 1.97, 64).astype(np.float32):
+        q = _dev(s * wave, torch.float32)
+        if solver == "pme":
+            ef, f = pm.create("real", batch=3), torch.empty_like(x)
+            pm.pme(x, q, 0.0, 1.0, 0.0, f, elec_field=ef)
+            got = np.abs(ef[axis].cpu().numpy().astype(np.float64)[odd])
+        else:
+            one = pm.create("real", 1.0, batch=1)
+            eps, contrib, dot, f = pm.create("real"), pm.create("real"), pm.create("real"), torch.empty_like(x)
+            call("hymd_update_field_force_q_gpe", pm.handle, dptr(x, torch.float32),
+                 dptr(torch.zeros(n, dtype=torch.int32, device="cuda"), torch.int32), dptr(q, torch.float32), n, 1,
+                 dptr(one, torch.float32), darr([1.0]), darr([0.0]), 0.0, 1.0, 1e-6, 0.6, 0, 10,
+                 dptr(eps, torch.float32), None, None, dptr(contrib, torch.float32), None,
+                 dptr(dot, torch.float32), None, dptr(f, torch.float32), None, None, None)
+            got = np.sqrt(dot.cpu().numpy().astype(np.float64)[odd])
+        errs.append(np.mean(got) / (4.0 * np.pi * float(s) / (dv * k)) - 1.0)
+    assert abs(np.mean(errs)) < 2e-8
