@@ -52,7 +52,8 @@ int fft_plan_init(FftPlan &plan, const Mesh &mesh);
 //                  in[T + t] = IFFT_x(V_t) (times -i k_y, -i k_z)
 //   real_v[t]      the grid of in[T + t] itself
 //   real2[t]       the grid of in2[t]
-// (k_y = kfy n_y, k_z = kfz n_z, zero on Nyquist planes); all times scale.
+// (k_y = kfy n_y, k_z = kfz n_z, zero on Nyquist planes, multiplied in FP32, or
+// with `wide` in FP64 and rounded once); all times scale.
 // Several systems of the same mesh and T follow each other in every list
 // (in: 2T spectra each), with their factors (kfy, kfz) in kf on the device.
 struct YzJob {
@@ -61,6 +62,7 @@ struct YzJob {
     const float2 *in = nullptr, *in2 = nullptr;
     float *force = nullptr, *real_v = nullptr, *real2 = nullptr;
     double kfy = 0.0, kfz = 0.0;
+    bool wide = false;
     float scale = 1.f;
 };
 

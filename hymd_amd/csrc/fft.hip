@@ -206,8 +206,12 @@ struct RealSplit {
     }
 };
 
-// -i kd v for a derivative factor kd
-__device__ __forceinline__ float2 mul_minus_i(float2 v, float kd) { return make_float2(kd * v.y, -kd * v.x); }
+// -i kd v for a derivative factor kd, in FP32 or (wide) in FP64
+__device__ __forceinline__ float2 mul_minus_i(float2 v, double kd, bool wide) {
+    if (wide) return make_float2((float)(kd * (double)v.y), (float)(-kd * (double)v.x));
+    const float k = (float)kd;
+    return make_float2(k * v.y, -k * v.x);
+}
 
 // Its inverse: Z'[m] = (X[m] + X*[nh-m]) + i conj(post[m]) (X[m] - X*[nh-m])
 __device__ __forceinline__ float2 real_join(const float2 *row, const float2 *post, int m, int nh) {
@@ -219,7 +223,7 @@ __device__ __forceinline__ float2 real_join(const float2 *row, const float2 *pos
 struct YzGrid {
     const float2 *src;
     float *dst;
-    bool dy, dz;
+    bool dy, dz, wide;
     double kfy, kfz;
 };
 
@@ -242,6 +246,7 @@ __device__ __forceinline__ YzGrid yz_grid(const YzArgs &a, int t, int d) {
                       : (kind == 3 ? a.job.real_v + (int64_t)t * a.g : a.job.force + (int64_t)(3 * t + kind) * a.g);
     q.dy = kind == 1;
     q.dz = kind == 2;
+    q.wide = a.job.wide;
     q.kfy = a.job.kf ? a.job.kf[sys].x : a.job.kfy;
     q.kfz = a.job.kf ? a.job.kf[sys].y : a.job.kfz;
     return q;
@@ -262,18 +267,17 @@ static YzArgs yz_args(const FftPlan &plan, const YzJob &job) {
 // the y line, so its factor commutes with the transform; both zero on their
 // Nyquist planes).
 struct YzFactor {
-    bool dy, dz;
+    bool dy, dz, wide;
     int y, my;
-    float kz;
-    double kfy;
+    double kfy, kz;
     __device__ YzFactor(const YzGrid &q, int y_, int m, int my_, int nh)
-        : dy(q.dy), dz(q.dz), y(y_), my(my_), kz(m == nh ? 0.f : (float)(q.kfz * m)), kfy(q.kfy) {}
+        : dy(q.dy), dz(q.dz), wide(q.wide), y(y_), my(my_), kfy(q.kfy), kz(m == nh ? 0.0 : q.kfz * m) {}
     __device__ float2 operator()(float2 v, int d) const {
         if (dy) {
             const int yy = y + d;
-            return mul_minus_i(v, 2 * yy == my ? 0.f : (float)(kfy * (2 * yy < my ? yy : yy - my)));
+            return mul_minus_i(v, 2 * yy == my ? 0.0 : kfy * (2 * yy < my ? yy : yy - my), wide);
         }
-        return dz ? mul_minus_i(v, kz) : v;
+        return dz ? mul_minus_i(v, kz, wide) : v;
     }
 };
 
@@ -426,7 +430,9 @@ __global__ void __launch_bounds__(NT, WPE)
                                                   [&](int kz, int y, float2 v) { dst[y * zh + kz] = v; });
 }
 
-template <int MY, int MZ, int NT, int WPE>
+// WIDE: of the job (in FP64 where the job asks, by a kernel of its own: as a
+// runtime choice it cost the 128^2 planes 2 %).
+template <int MY, int MZ, int NT, int WPE, bool WIDE>
 __global__ void __launch_bounds__(NT, WPE) c2r_yz_plane_kernel_fixed(YzArgs a, PlaneFixed<MY, MZ, NT, WPE> g) {
     extern __shared__ float2 smem[];
     constexpr int my = MY, mz = MZ, nh = MZ / 2, zh = MZ / 2 + 1;
@@ -439,7 +445,7 @@ __global__ void __launch_bounds__(NT, WPE) c2r_yz_plane_kernel_fixed(YzArgs a, P
         float2 w = src[y * zh + kz];
         if (q.dy) {  // row y: k_y, zero on the Nyquist row
             const int ny = 2 * y < my ? y : y - my;
-            w = mul_minus_i(w, 2 * y == my ? 0.f : (float)(q.kfy * ny));
+            w = mul_minus_i(w, 2 * y == my ? 0.0 : q.kfy * ny, WIDE);
         }
         return w;
     });
@@ -451,8 +457,8 @@ __global__ void __launch_bounds__(NT, WPE) c2r_yz_plane_kernel_fixed(YzArgs a, P
         const int p = nh - m;
         float2 xm = row[m], xp = row[p];
         if (q.dz) {  // column kz: k_z, zero on the Nyquist column
-            xm = mul_minus_i(xm, 2 * m == mz ? 0.f : (float)(q.kfz * m));
-            xp = mul_minus_i(xp, 2 * p == mz ? 0.f : (float)(q.kfz * p));
+            xm = mul_minus_i(xm, 2 * m == mz ? 0.0 : q.kfz * m, WIDE);
+            xp = mul_minus_i(xp, 2 * p == mz ? 0.0 : q.kfz * p, WIDE);
         }
         const float2 sm = cadd(xm, cconj(xp));
         const float2 df = cmul(cconj(s.post[m]), csub(xm, cconj(xp)));
@@ -467,11 +473,13 @@ __global__ void __launch_bounds__(NT, WPE) c2r_yz_plane_kernel_fixed(YzArgs a, P
 template <class G>
 static constexpr auto r2c_plane(const G &) { return &r2c_zy_plane_kernel<G>; }
 template <class G>
-static constexpr auto c2r_plane(const G &) { return &c2r_yz_plane_kernel<G>; }
+static constexpr auto c2r_plane(const G &, bool) { return &c2r_yz_plane_kernel<G>; }
 template <int MY, int MZ, int NT, int WPE>
 static constexpr auto r2c_plane(const PlaneFixed<MY, MZ, NT, WPE> &) { return &r2c_zy_plane_kernel_fixed<MY, MZ, NT, WPE>; }
 template <int MY, int MZ, int NT, int WPE>
-static constexpr auto c2r_plane(const PlaneFixed<MY, MZ, NT, WPE> &) { return &c2r_yz_plane_kernel_fixed<MY, MZ, NT, WPE>; }
+static constexpr auto c2r_plane(const PlaneFixed<MY, MZ, NT, WPE> &, bool wide) {
+    return wide ? &c2r_yz_plane_kernel_fixed<MY, MZ, NT, WPE, true> : &c2r_yz_plane_kernel_fixed<MY, MZ, NT, WPE, false>;
+}
 
 // ---------------------------------------------------------------------------
 // line passes: z rows (contiguous) and strided lines
@@ -846,9 +854,10 @@ int fft_yz_multi(const FftPlan &plan, const YzJob &job, float2 *tmp, hipStream_t
         const int blocks = plan.mesh.mx * grids;
         return with_plane(plan, blocks, true, [&](auto g, int threads) -> int {
             using G = decltype(g);
-            static bool done = false;
-            if (plan.lds_plane > 64 * 1024) HYMD_TRY(lds_opt_in(c2r_plane(g), done));
-            c2r_plane(g)<<<blocks, threads, plan.lds_plane, s>>>(a, g);
+            static bool done[2] = {false, false};
+            const auto kernel = c2r_plane(g, job.wide);
+            if (plan.lds_plane > 64 * 1024) HYMD_TRY(lds_opt_in(kernel, done[job.wide]));
+            kernel<<<blocks, threads, plan.lds_plane, s>>>(a, g);
             HYMD_HIP(hipGetLastError());
             return HYMD_OK;
         });

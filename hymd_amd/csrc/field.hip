@@ -1077,7 +1077,8 @@ extern "C" int hymd_readout(hymd_pm *pm, const float *grid, const float *x, int6
 
 // The y-z passes of the x-inverse spectra that kspace_pass left in pm->grad:
 // the force grids, optionally the potentials v and, from phix, the densities.
-static int yz_passes(hymd_pm *pm, int T, float *force_mesh, float *v, const float2 *phix, float *phi) {
+static int yz_passes(hymd_pm *pm, int T, float *force_mesh, float *v, const float2 *phix, float *phi,
+                     bool wide = false) {
     const KGeom g = kgeom(pm);
     YzJob job;
     job.T = T;
@@ -1088,6 +1089,7 @@ static int yz_passes(hymd_pm *pm, int T, float *force_mesh, float *v, const floa
     job.real2 = phi;
     job.kfy = g.kfac[1];
     job.kfz = g.kfac[2];
+    job.wide = wide;
     const int tmp = fft_yz_tmp(pm->fft, job);
     if (tmp) HYMD_TRY(pm->cscratch.reserve(sizeof(float2) * pm->mesh.gc * tmp));
     return fft_yz_multi(pm->fft, job, (float2 *)pm->cscratch.ptr, pm->stream);
@@ -1095,9 +1097,9 @@ static int yz_passes(hymd_pm *pm, int T, float *force_mesh, float *v, const floa
 
 // The field -grad psi (3 grids) and, if not null, psi of the charge grid rho:
 // psi = p.four_pi_elec H rho / |k|^2; energy partials (*nparts of them).  The
-// y-z pass forms E_y, E_z and psi from psi's x-inverse spectrum.
+// y-z pass forms E_y, E_z and psi from psi's x-inverse spectrum (wide: YzJob).
 static int poisson(hymd_pm *pm, const float *rho, const PmeK &p, float *field, float *psi, double *partials,
-                   int *nparts) {
+                   int *nparts, bool wide = false) {
     hipStream_t s = pm->stream;
     float2 *spec = (float2 *)pm->spec.ptr, *out = (float2 *)pm->grad.ptr;
     const KGeom g = kgeom(pm);
@@ -1119,7 +1121,7 @@ static int poisson(hymd_pm *pm, const float *rho, const PmeK &p, float *field, f
         HYMD_HIP(hipGetLastError());
         HYMD_TRY(fft_inverse_x(pm->fft, out, 2, s));
     }
-    return yz_passes(pm, 1, field, psi, nullptr, nullptr);
+    return yz_passes(pm, 1, field, psi, nullptr, nullptr, wide);
 }
 
 // The x transforms and the k-space pass of p.T types from the spectra in
@@ -1809,7 +1811,7 @@ extern "C" int hymd_update_field_force_q_gpe(hymd_pm *pm, const float *x, const 
     gpe_kspace_kernel<<<kb, kBlock, 0, s>>>(spec, grad, g, 0, 1, s2, inv_g);
     HYMD_HIP(hipGetLastError());
     HYMD_TRY(fft_inverse_x(pm->fft, grad, 2, s));
-    HYMD_TRY(yz_passes(pm, 1, eta, nullptr, nullptr, nullptr));
+    HYMD_TRY(yz_passes(pm, 1, eta, nullptr, nullptr, nullptr, true));
     gpe_eta_kernel<<<eb, kBlock, 0, s>>>(eta, phi_eps, G);
     HYMD_HIP(hipGetLastError());
     // 5. polarisation charges from the caller's previous grid
@@ -1839,7 +1841,7 @@ extern "C" int hymd_update_field_force_q_gpe(hymd_pm *pm, const float *x, const 
         HYMD_TRY(ev.create());
         for (int k = 0;; ++k) {
             if (k < max_iter) {
-                HYMD_TRY(poisson(pm, tmp, pk, E, nullptr, nullptr, &unused));
+                HYMD_TRY(poisson(pm, tmp, pk, E, nullptr, nullptr, &unused, true));
                 gpe_pol_kernel<<<eb, kBlock, 0, s>>>(eta, E, phq, pol, tmp, G, (float)pol_mixing, state, part);
                 gpe_check_kernel<<<1, kBlock, 0, s>>>(part, eb, conv_type, conv_crit, state);
                 HYMD_HIP(hipGetLastError());
@@ -1858,7 +1860,7 @@ extern "C" int hymd_update_field_force_q_gpe(hymd_pm *pm, const float *x, const 
     const double eps0_inv = 4.0 * M_PI * coulomb_constant;
     pk.four_pi_elec = eps0_inv;
     float *psi_g = psi ? psi : psi_i;
-    HYMD_TRY(poisson(pm, tmp, pk, E, psi_g, nullptr, &unused));
+    HYMD_TRY(poisson(pm, tmp, pk, E, psi_g, nullptr, &unused, true));
     // 7. |E|^2, contrib, V_t and the energy partials
     gpe_vbar_kernel<<<eb, kBlock, 0, s>>>(E, psi_g, phi_eps, den, p, (float)(0.5 / eps0_inv), G, elec_field_contrib,
                                           elec_dot, vb, part);
@@ -1870,7 +1872,7 @@ extern "C" int hymd_update_field_force_q_gpe(hymd_pm *pm, const float *x, const 
     gpe_kspace_kernel<<<kb, kBlock, 0, s>>>(spec, grad, g, 3, T, s2, inv_g);
     HYMD_HIP(hipGetLastError());
     HYMD_TRY(fft_inverse_x(pm->fft, grad, 2 * T, s));
-    HYMD_TRY(yz_passes(pm, T, fm, nullptr, nullptr, nullptr));
+    HYMD_TRY(yz_passes(pm, T, fm, nullptr, nullptr, nullptr, true));
     HYMD_TRY(sort_particles(pm, x, types, nullptr, n));
     HYMD_TRY(readout_sorted(pm, 3, T, fm, elec_forces, false));
     if (energy) *energy = cell_volume(pm) * (0.5 / eps0_inv) * e_sum;

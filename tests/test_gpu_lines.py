@@ -306,7 +306,7 @@ def test_xline_width_takes_effect(hip, mesh, T, other, own):
         assert rms_rel(a.cpu().numpy(), b.cpu().numpy()) < 1e-6
 
 
-@pytest.mark.parametrize("solver,axis", [("pme", 0), ("gpe", 0)])
+@pytest.mark.parametrize("solver,axis", [("pme", 0), ("gpe", 0), ("gpe", 1), ("gpe", 2)])
 def test_derivative_factor_in_fp64(hip, solver, axis):
     """The electric field of a charge density cos(2 k x) on eight points, whose
     transforms are exact (factors of 1 and i), in a box whose k rounds to FP32
