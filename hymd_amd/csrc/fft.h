@@ -79,7 +79,8 @@ int fft_inverse_x(const FftPlan &plan, float2 *data, int batch, hipStream_t s);
 int fft_c2r_yz(const FftPlan &plan, float2 *in, float *out, int batch, float scale, hipStream_t s);
 int fft_c2r(const FftPlan &plan, float2 *data, float *out, int batch, float scale, hipStream_t s);
 // The grids of `job`.  Where the planes do not fit in LDS, tmp holds one half
-// spectrum per grid made (fft_yz_tmp of them; 0: none needed).
+// spectrum for each of the grids made at a time (fft_yz_tmp of them; 0: none
+// needed).
 int fft_yz_multi(const FftPlan &plan, const YzJob &job, float2 *tmp, hipStream_t s);
 int fft_yz_tmp(const FftPlan &plan, const YzJob &job);
 

@@ -229,9 +229,10 @@ struct YzGrid {
 
 // kinds: the job's grids of one type in order, 3 bits each (0-2 gradient
 // along x, y, z; 3 real_v; 4 real2)
+// grid0: the first grid of a launch that takes some of them (the line passes).
 struct YzArgs {
     YzJob job;
-    int nkinds, kinds;
+    int nkinds, kinds, grid0;
     int64_t g, gc;
 };
 
@@ -253,7 +254,7 @@ __device__ __forceinline__ YzGrid yz_grid(const YzArgs &a, int t, int d) {
 }
 
 static YzArgs yz_args(const FftPlan &plan, const YzJob &job) {
-    YzArgs a{job, 0, 0, plan.mesh.g, plan.mesh.gc};
+    YzArgs a{job, 0, 0, 0, plan.mesh.g, plan.mesh.gc};
     auto add = [&](int kind) { a.kinds |= kind << (3 * a.nkinds++); };
     if (job.force)
         for (int k = 0; k < 3; ++k) add(k);
@@ -531,7 +532,7 @@ __global__ void __launch_bounds__(kBlock) r2c_z_kernel(const float *__restrict__
 }
 
 // z pass of a YzJob, half spectrum -> real: block (grid, W rows), the
-// y-transformed spectra in tmp, grid t nkinds + d.
+// y-transformed spectra in tmp, grid t nkinds + d at tmp + (it - grid0) gc.
 template <class G>
 __global__ void __launch_bounds__(kBlock) c2r_z_kernel(const float2 *__restrict__ tmp, YzArgs a, int64_t rows,
                                                        int blocks, G g) {
@@ -540,11 +541,11 @@ __global__ void __launch_bounds__(kBlock) c2r_z_kernel(const float2 *__restrict_
     for (int i = threadIdx.x; i < g.nh - 1; i += kBlock) tw[i] = g.twz[i];
     for (int i = threadIdx.x; i < g.zh; i += kBlock) post[i] = g.post[i];
     const int flat = (int)xcd_block(blockIdx.x, gridDim.x);
-    const int grid = flat / blocks, t = grid / a.nkinds;
+    const int local = flat / blocks, grid = a.grid0 + local, t = grid / a.nkinds;
     const YzGrid q = yz_grid(a, t, grid - t * a.nkinds);
-    const int64_t row0 = (int64_t)(flat - grid * blocks) * g.W;
+    const int64_t row0 = (int64_t)(flat - local * blocks) * g.W;
     const int wv = (int)(rows - row0 < g.W ? rows - row0 : g.W);
-    const float2 *src = tmp + (int64_t)grid * a.gc + row0 * g.zh;
+    const float2 *src = tmp + (int64_t)local * a.gc + row0 * g.zh;
     float2 *dst = reinterpret_cast<float2 *>(q.dst) + row0 * g.nh;
     const int total = wv * g.zh;
     for (int i0 = threadIdx.x; i0 < g.W * g.zh; i0 += kBlock * kLoadBatch) {
@@ -634,16 +635,17 @@ __global__ void __launch_bounds__(G::threads) fft_strided_kernel(float2 *__restr
     });
 }
 
-// Out-of-place inverse y pass of a YzJob into tmp, grid t nkinds + d.
+// Out-of-place inverse y pass of a YzJob into tmp, laid out as c2r_z_kernel reads it.
 template <class G>
 __global__ void __launch_bounds__(G::threads) fft_y_multi_kernel(float2 *__restrict__ tmp, YzArgs a, Strided q, G g) {
     extern __shared__ float2 smem[];
     float2 *tw = smem, *A = tw + g.n;
     for (int i = threadIdx.x; i < g.n - 1; i += G::nt()) tw[i] = g.tw[i];
     const int flat = (int)xcd_block(blockIdx.x, gridDim.x);
-    const int grid = flat / q.blocks, line0 = (flat - grid * q.blocks) * q.W, t = grid / a.nkinds;
+    const int local = flat / q.blocks, line0 = (flat - local * q.blocks) * q.W;
+    const int grid = a.grid0 + local, t = grid / a.nkinds;
     const YzGrid y = yz_grid(a, t, grid - t * a.nkinds);
-    float2 *dst = tmp + (int64_t)grid * a.gc;
+    float2 *dst = tmp + (int64_t)local * a.gc;
     const int wv = min(q.W, q.nlines - line0);
     line_first<1, false>(A, g.lines(wv), g.axis(), [&](int l, int e) {
         const int line = line0 + l, x = divq(line, q.inv_inner), kz = line - x * q.inner;
@@ -830,17 +832,24 @@ int fft_r2c_real(const FftPlan &plan, const float *in, float2 *out, int batch, h
     return fft_forward_x(plan, out, batch, s);
 }
 
+// The line passes take this many of a job's grids at a time: all, up to five
+// per type, while that is 4 GB of scratch at most, then as many as 4 GB hold and
+// at least one per type.  Several goes cost the ends of their launches: 256^3,
+// six types, force grids 2072 us, one per type at a time 2146.
 int fft_yz_tmp(const FftPlan &plan, const YzJob &job) {
-    return plan.lds_plane ? 0 : job.T * job.systems * yz_args(plan, job).nkinds;
+    if (plan.lds_plane) return 0;
+    const int64_t some = (int64_t(4) << 30) / ((int64_t)sizeof(float2) * plan.mesh.gc);
+    const int64_t types = (int64_t)job.T * job.systems;
+    return (int)std::min(std::max(some, types), types * yz_args(plan, job).nkinds);
 }
 
-// The z pass of a job whose y-transformed spectra are in tmp.
-static int launch_z_inverse(const FftPlan &plan, const YzArgs &a, const float2 *tmp, hipStream_t s) {
+// The z pass of `grids` of a job's grids, whose y-transformed spectra are in tmp.
+static int launch_z_inverse(const FftPlan &plan, const YzArgs &a, int grids, const float2 *tmp, hipStream_t s) {
     const int64_t rows = (int64_t)plan.mesh.mx * plan.mesh.my;
     const int blocks = (int)((rows + plan.wz - 1) / plan.wz);
     return with_rows(plan, [&](auto g) -> int {
         using G = decltype(g);
-        c2r_z_kernel<G><<<blocks * a.job.T * a.job.systems * a.nkinds, kBlock, z_lds(plan), s>>>(tmp, a, rows, blocks, g);
+        c2r_z_kernel<G><<<blocks * grids, kBlock, z_lds(plan), s>>>(tmp, a, rows, blocks, g);
         HYMD_HIP(hipGetLastError());
         return HYMD_OK;
     });
@@ -863,14 +872,20 @@ int fft_yz_multi(const FftPlan &plan, const YzJob &job, float2 *tmp, hipStream_t
         });
     }
     HYMD_REQUIRE(tmp, "planes that do not fit in LDS need the line passes' scratch");
-    Strided q = strided_lines(plan, 1, 1);
-    HYMD_TRY(with_strided(plan, 1, q.W, [&](auto g) -> int {
-        using G = decltype(g);
-        fft_y_multi_kernel<G><<<q.blocks * grids, G::threads, strided_lds(plan.ly, q.W), s>>>(tmp, a, q, g);
-        HYMD_HIP(hipGetLastError());
-        return HYMD_OK;
-    }));
-    return launch_z_inverse(plan, a, tmp, s);
+    const Strided q = strided_lines(plan, 1, 1);
+    const int step = fft_yz_tmp(plan, job);
+    YzArgs b = a;
+    for (b.grid0 = 0; b.grid0 < grids; b.grid0 += step) {
+        const int some = std::min(step, grids - b.grid0);
+        HYMD_TRY(with_strided(plan, 1, q.W, [&](auto g) -> int {
+            using G = decltype(g);
+            fft_y_multi_kernel<G><<<q.blocks * some, G::threads, strided_lds(plan.ly, q.W), s>>>(tmp, b, q, g);
+            HYMD_HIP(hipGetLastError());
+            return HYMD_OK;
+        }));
+        HYMD_TRY(launch_z_inverse(plan, b, some, tmp, s));
+    }
+    return HYMD_OK;
 }
 
 int fft_c2r_yz(const FftPlan &plan, float2 *in, float *out, int batch, float scale, hipStream_t s) {
@@ -881,7 +896,7 @@ int fft_c2r_yz(const FftPlan &plan, float2 *in, float *out, int batch, float sca
     job.scale = scale;
     if (plan.lds_plane) return fft_yz_multi(plan, job, nullptr, s);
     HYMD_TRY(launch_strided(plan, in, batch, 1, 1.f, s));  // y in place, then the z pass from there
-    return launch_z_inverse(plan, yz_args(plan, job), in, s);
+    return launch_z_inverse(plan, yz_args(plan, job), batch, in, s);
 }
 
 int fft_c2r(const FftPlan &plan, float2 *data, float *out, int batch, float scale, hipStream_t s) {

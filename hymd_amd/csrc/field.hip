@@ -697,7 +697,6 @@ struct hymd_pm {
     DevBuf grad;      // max(3 max_types, 4) x Gc complex
     DevBuf cscratch;  // complex scratch of the line passes (and of hymd_fft_c2r)
     DevBuf gpe_state; // the variable-dielectric iteration's GpeState
-    DevBuf phix;      // x-inverse filtered spectra, when the densities are asked for
     DevBuf rscratch;  // 3 x G float (PME field when the caller passes none)
     DevBuf partials;  // energy partial sums
     DevBuf result;    // reduced doubles
@@ -723,7 +722,7 @@ struct hymd_pm {
 
 uint64_t hymd::pm_generation(const hymd_pm *pm) {
     uint64_t g = pm->box_version;
-    for (const DevBuf *b : {&pm->paint, &pm->spec, &pm->grad, &pm->cscratch, &pm->phix, &pm->gpe_state, &pm->rscratch, &pm->partials,
+    for (const DevBuf *b : {&pm->paint, &pm->spec, &pm->grad, &pm->cscratch, &pm->gpe_state, &pm->rscratch, &pm->partials,
                             &pm->result, &pm->mpart, &pm->keys, &pm->perm, &pm->xs, &pm->ws, &pm->counts,
                             &pm->start, &pm->tiles})
         g += b->allocs;
@@ -1188,11 +1187,7 @@ static int update_field_impl(hymd_pm *pm, const float *x, const int32_t *types, 
     p.want_energy = energy ? 1 : 0;
     // 2. z + y forward passes; the x-line pass; the y-z pass writes the grids
     HYMD_TRY(fft_r2c_zy(pm->fft, rho, spec, T, s));
-    float2 *phix = nullptr;
-    if (phi) {
-        HYMD_TRY(pm->phix.reserve(sizeof(float2) * m.gc * T));
-        phix = (float2 *)pm->phix.ptr;
-    }
+    float2 *phix = phi ? (float2 *)pm->grad.ptr + 2 * T * m.gc : nullptr;  // of grad's 3T spectra kspace_pass fills 2T
     int nb = 0;
     HYMD_TRY(kspace_pass(pm, p, false, (float2 *)phi_fourier, phix, energy ? (double *)pm->partials.ptr : nullptr, &nb));
     HYMD_TRY(yz_passes(pm, T, force_mesh, v_ext, phix, phi));
