@@ -4,6 +4,8 @@ Tolerances: the int64 fixed-point density grid is compared bit for bit; FP32
 FFT / forces against the FP64 oracle within the north-star bound of 1e-4
 relative RMS (tighter where the data allow, stated per test).
 """
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -252,15 +254,16 @@ def test_drop_in_field_surface(hip):
                                     ((128, 40, 24), 4), ((128, 24, 20), 2), ((128, 20, 16), 3), ((128, 16, 12), 1),
                                     ((160, 20, 16), 3), ((160, 16, 24), 1),
                                     ((16, 128, 128), 4), ((8, 160, 160), 2),
-                                    # long x lines with many types: 8 lines per workgroup of 1024 threads
+                                    # long x lines with many types (256 points, five: 8 lines of 1024 threads)
                                     ((192, 16, 16), 6), ((256, 12, 10), 5), ((512, 8, 8), 4), ((160, 24, 20), 7)])
 def test_fused_xline_pass_equals_unfused(hip, mesh, T):
     """The force-grid-only update (forward x, k-space and inverse x passes in
-    one kernel, -i k_y and -i k_z applied in the y-z plane pass) against the
-    unfused passes (-i k_d V_t formed in k-space, then three full inverse
-    transforms per type), which run when v_ext is requested.  The same
-    operator, applied in a different order, so the grids agree to FP32
-    rounding, not bit for bit."""
+    one kernel, -i k_y and -i k_z applied in the y-z pass) against the separate
+    passes, which the moments' force grids take for every mesh (transforms of all
+    three axes, the k-space pass by itself, inverse x transforms), and the FP64
+    oracle.  The same operator with other radices along x, so the grids agree to
+    FP32 rounding, not bit for bit."""
+    from hymd_amd._lib import call, darr, dptr
     rng = np.random.default_rng(5)
     box = (6.0, 7.5, 5.0)
     n = 6000
@@ -273,13 +276,23 @@ def test_fused_xline_pass_equals_unfused(hip, mesh, T):
     xd, td = _dev(x, torch.float32), _dev(types, torch.int32)
     f1 = pm.create("real", batch=(T, 3))
     f2 = pm.create("real", batch=(T, 3))
-    v = pm.create("real", batch=T)
     e1 = pm.field_update(xd, td, T, A, b, 0.3, [1.0] * T, 0.45, f1, want_energy=True)
-    e2 = pm.field_update(xd, td, T, A, b, 0.3, [1.0] * T, 0.45, f2, v_ext=v, want_energy=True)
+    npair = T * (T + 1) // 2
+    mom = np.zeros(2 * npair + T)
+    call("hymd_field_moments", pm.handle, dptr(xd, torch.float32), dptr(td, torch.int32), n, T, darr([1.0] * T), 0.45,
+         mom.ctypes.data_as(ctypes.POINTER(ctypes.c_double)), darr(np.ravel(A)), darr(b), dptr(f2, torch.float32))
+    # V (1/2 sum A P + b . phi~(0) + c0), the pairs t < s counted twice
+    twice = np.where(np.eye(T)[np.triu_indices(T)] > 0, 0.5, 1.0)
+    e2 = np.prod(box) * (np.sum(twice * A[np.triu_indices(T)] * mom[:npair]) + b @ mom[2 * npair:] + 0.3)
     a1, a2 = f1.cpu().numpy(), f2.cpu().numpy()
     assert np.abs(a1 - a2).max() <= 1e-6 * np.abs(a2).max()
     assert rms_rel(a1, a2) < 2e-7
-    assert e1 == pytest.approx(e2, rel=1e-9)
+    # the update rounds the factor H/G and its product with the spectrum to FP32,
+    # 2^-24 each at most and twice in a square; the moments do not
+    assert e1 == pytest.approx(e2, rel=4 * 2.0 ** -24)
+    ref = F.update_field(x.astype(np.float64), types, T, mesh, box, 0.45, F.Quadratic(A, b, 0.3))
+    want = np.array([[ref["force_mesh"][t][d] for d in range(3)] for t in range(T)])
+    assert rms_rel(a1, want) < 1e-6
 
 
 @pytest.mark.parametrize("mesh,T", [((20, 24, 18), 3), ((16, 16, 16), 2), ((12, 10, 8), 5), ((24, 20, 30), 8),

@@ -42,7 +42,7 @@ def test_line_plans_vs_numpy(hip, mesh):
 
 @pytest.mark.parametrize("mesh", [(4, 6, 8), (6, 4, 6), (18, 10, 12), (16, 30, 20), (30, 16, 10), (128, 8, 6),
                                   (150, 6, 8), (96, 10, 16), (256, 6, 4), (64, 20, 18), (8, 100, 100), (4, 150, 160),
-                                  (6, 192, 200)])
+                                  (6, 192, 200), (160, 6, 8), (192, 6, 8), (216, 6, 8), (240, 6, 8)])
 @pytest.mark.parametrize("T", [1, 2, 3, 4, 5, 6, 7, 8, 9])
 def test_field_pass_matches_oracle(hip, mesh, T):
     """Force grids, densities, their spectra, potentials and energy of one
@@ -75,6 +75,40 @@ def test_field_pass_matches_oracle(hip, mesh, T):
     assert e == pytest.approx(F.field_energy(ref["phi"], ham, mesh, box), rel=1e-6)
 
 
+# lines enough (4160) for the widths that small meshes halve: 8 lines of 384 to
+# 512 threads, 4 lines, and one line of one and of two types
+@pytest.mark.parametrize("mesh,T", [((180, 64, 128), 4), ((200, 64, 128), 3), ((240, 64, 128), 2), ((256, 64, 128), 4),
+                                    ((160, 64, 128), 5), ((144, 64, 128), 4), ((100, 64, 128), 8), ((900, 10, 8), 1),
+                                    ((720, 10, 8), 2)])
+def test_field_pass_at_full_width(hip, mesh, T):
+    test_field_pass_matches_oracle(hip, mesh, T)
+
+
+@pytest.mark.parametrize("mesh", [(6, 10, 8), (90, 12, 10), (160, 8, 6), (180, 64, 128), (216, 10, 8), (240, 64, 128),
+                                  (256, 8, 10), (900, 6, 8)])
+def test_pme_pass_matches_oracle(hip, mesh):
+    """Field, potential and energy of the PME solve against the FP64 oracle at
+    the x edges where its x-line pass changes (1e-6 of each one's RMS; an FP32
+    transform's error is 2e-7 there)."""
+    from hymd_amd.field import ParticleMesh
+    rng = np.random.default_rng(sum(mesh))
+    box = np.array(mesh) * 0.25
+    n = 3000
+    x = (rng.uniform(0, 1, (n, 3)) * box).astype(np.float32)
+    q = np.where(np.arange(n) % 2, 1.0, -1.0)
+    ref = F.update_field_force_q(x.astype(np.float64), q, mesh, box, 0.4, 138.9, 45.0)
+    pm = ParticleMesh(mesh, box, 1)
+    f, ef = torch.empty((n, 3), dtype=torch.float32, device="cuda"), pm.create("real", batch=3)
+    psi, rho = pm.create("real"), pm.create("real")
+    e = pm.pme(_dev(x, torch.float32), _dev(q, torch.float32), 0.4, 138.9 / 45.0, 0.0, f, phi_q=rho, psi=psi,
+               elec_field=ef, want_energy=True)
+    assert rms_rel(psi.cpu().numpy(), ref["psi"]) < 1e-6
+    for d in range(3):
+        assert rms_rel(ef[d].cpu().numpy(), ref["elec_field"][d]) < 1e-6
+    assert rms_rel(f.cpu().numpy(), ref["forces"]) < 1e-6
+    assert e == pytest.approx(F.field_q_energy(ref["phi_q"], ref["psi"], 0.0, mesh, box), rel=1e-6)
+
+
 def test_edges_refused(hip):
     from hymd_amd._lib import HymdError
     from hymd_amd.field import ParticleMesh
@@ -88,8 +122,10 @@ def test_edges_refused(hip):
 @pytest.mark.parametrize("n", [(1 << 20), (1 << 20) + 1, (1 << 20) + 1027])
 @pytest.mark.parametrize("ordered", [False, True])
 def test_binning_of_large_inputs(hip, n, ordered):
-    """Painted grids of the sorted path equal the scatter paint's bit for bit;
-    zero-weight particles and one crowded row among them."""
+    """Painted grids of the sorted path equal the scatter paint's bit for bit,
+    one crowded row among them; and with weights, nine in ten of them and all of
+    8192 successive particles zero (those are not binned: whole wavefronts
+    and workgroups of them, and such that start with one)."""
     from hymd_amd.field import ParticleMesh
     mesh, box, T = (18, 20, 16), (4.5, 5.0, 4.0), 2
     rng = np.random.default_rng(n + ordered)
@@ -105,6 +141,52 @@ def test_binning_of_large_inputs(hip, n, ordered):
     scat = torch.zeros((T,) + mesh, dtype=torch.int64, device="cuda")
     pm.paint_fixed(xd, td, T, out=scat, accumulate=True)
     assert torch.equal(grid.to(torch.int64), scat)
+    w = rng.uniform(-1.0, 1.0, n) * (rng.random(n) < 0.1)
+    w[5000: 5000 + 8192] = 0.0
+    wd = _dev(w, torch.float32)
+    scat = torch.zeros((1,) + mesh, dtype=torch.int64, device="cuda")
+    pm.paint_fixed(xd, None, 1, weights=wd, out=scat, accumulate=True)
+    assert torch.equal(pm.paint_fixed(xd, None, 1, weights=wd), scat)
+
+
+@pytest.mark.parametrize("ordered", [False, True])
+def test_batch_of_many_particles(hip, ordered):
+    """A batch of more than 2^20 particles (keys ranked per workgroup), replicas
+    that end within a wavefront or a workgroup and an empty one: moments and
+    forces of each equal those of the replica alone, bit for bit."""
+    from hymd_amd.batch import ReplicaBatch
+    from hymd_amd.field import ParticleMesh
+    counts = np.array([400001, 350003, 0, 63, 300007, 90001])
+    meshes = np.array([[32, 24, 20], [24, 24, 24], [16, 16, 16], [16, 16, 16], [32, 24, 20], [20, 16, 18]])
+    boxes = meshes * 0.4
+    rng = np.random.default_rng(7 + ordered)
+    xs, ts = [], []
+    for c, m, L in zip(counts, meshes, boxes):
+        x = rng.uniform(0, 1, (c, 3)) * L
+        if ordered:
+            cell = (x / 0.4).astype(np.int64)
+            x = x[np.lexsort((cell[:, 2], cell[:, 1], cell[:, 0]))]
+        xs.append(_dev(x, torch.float32))
+        ts.append(_dev(rng.integers(0, 2, c), torch.int32))
+    b = ReplicaBatch(meshes, boxes, counts, 2)
+    R, kappa, sigma = len(counts), np.full(len(counts), 0.05), np.full(len(counts), 0.5)
+    chi = np.zeros((R, 2, 2))
+    chi[:, 0, 1] = chi[:, 1, 0] = 20.0
+    x, t = torch.cat(xs), torch.cat(ts)
+    got = b.moments(x, t, sigma)
+    forces = b.energy_forces_and_gradients(x, t, chi, kappa, sigma)[4]
+    rho0 = counts / np.prod(boxes, axis=1)
+    A = b.coupling(chi, kappa, rho0)
+    first = np.concatenate([[0], np.cumsum(counts)])
+    for r in np.flatnonzero(counts):
+        pm = ParticleMesh(tuple(int(v) for v in meshes[r]), boxes[r], 2)
+        grids, P, phi0 = _moment_grids(pm, xs[r], ts[r], 2, A[r], np.zeros(2), float(sigma[r]))
+        np.testing.assert_array_equal(got[r][0], P)
+        np.testing.assert_array_equal(got[r][2], phi0)
+        f = torch.empty_like(xs[r])
+        pm.readout_forces(xs[r], ts[r], 2, grids, f)
+        assert torch.equal(forces[first[r]: first[r + 1]], f)
+    b.close()
 
 
 # no iteration, one, several; a mesh whose x lines have no x-line pass (Mx = 4)
@@ -151,33 +233,48 @@ def test_dielectric_iteration_counts(hip, mesh, crit, conv):
 
 @pytest.mark.parametrize("bad", [-1, 40])
 @pytest.mark.parametrize("energies", [False, True])
-def test_bonded_index_out_of_range(hip, bad, energies):
+@pytest.mark.parametrize("term", ["bonds", "angles", "dihedrals"])
+def test_bonded_index_out_of_range(hip, bad, energies, term):
     """The stateless kernels find a bad index while the forces are enqueued:
-    the call is refused, the forces stay as they were, the next call works."""
-    import ctypes
+    the call is refused, forces, dipoles, transfer matrices and energies stay as
+    they were, the next call works."""
     from hymd_amd import _lib
-    n, m = 40, 39
-    x = torch.rand((n, 3), device="cuda", dtype=torch.float32)
-    a = torch.arange(m, device="cuda", dtype=torch.int32)
-    b = a + 1
-    k, r0 = torch.ones(m, device="cuda", dtype=torch.float64), torch.full((m,), 0.1, device="cuda", dtype=torch.float64)
+    n, m = 40, 37
+    real = torch.float32
+    x = torch.rand((n, 3), generator=torch.Generator().manual_seed(3), dtype=real).cuda()
+    idx = [torch.arange(m, device="cuda", dtype=torch.int32) + j for j in range(4)]
+    par = [torch.full((m,), v, device="cuda", dtype=torch.float64) for v in (0.1, 1.0)]
+    coeff = torch.rand((m, 6, 5), generator=torch.Generator().manual_seed(4), dtype=real).cuda()
+    dtype, last = torch.ones(m, device="cuda", dtype=torch.int32), torch.ones(m, device="cuda", dtype=torch.int32)
     box = (ctypes.c_double * 3)(2.0, 2.0, 2.0)
-    e, pr = ctypes.c_double(-7.0), (ctypes.c_double * 3)()
+    e, pr, clamped = ctypes.c_double(-7.0), (ctypes.c_double * 3)(-7.0, -7.0, -7.0), ctypes.c_int64(-7)
+    out = [torch.full(shape, 5.0, device="cuda", dtype=real) for shape in ((n, 3), (m, 4, 3), (m, 6, 3, 3))]
 
-    def bonds(second, f):
-        _lib.call("hymd_cbf", f.data_ptr(), x.data_ptr(), n, box, a.data_ptr(), second.data_ptr(), r0.data_ptr(),
-                  k.data_ptr(), m, _lib.HYMD_F32, ctypes.byref(e) if energies else None,
-                  pr if energies else None, None)
+    def evaluate(members):
+        p = [v.data_ptr() for v in members]
+        energy = ctypes.byref(e) if energies else None
+        if term == "dihedrals":
+            _lib.call("hymd_cdf", out[0].data_ptr(), x.data_ptr(), out[1].data_ptr(), out[2].data_ptr(), n, box, *p,
+                      coeff.data_ptr(), dtype.data_ptr(), last.data_ptr(), m, 1, _lib.HYMD_F32, energy,
+                      ctypes.byref(clamped) if energies else None, None)
+        else:
+            _lib.call("hymd_cbf" if term == "bonds" else "hymd_caf", out[0].data_ptr(), x.data_ptr(), n, box, *p,
+                      par[0].data_ptr(), par[1].data_ptr(), m, _lib.HYMD_F32, energy, pr if energies else None, None)
 
-    f = torch.full((n, 3), 5.0, device="cuda", dtype=torch.float32)
-    wrong = b.clone()
-    wrong[7] = bad
+    members = idx[: {"bonds": 2, "angles": 3, "dihedrals": 4}[term]]
+    wrong = [v.clone() for v in members]
+    wrong[-1][7] = bad
     torch.cuda.synchronize()
     with pytest.raises(_lib.HymdError):
-        bonds(wrong, f)
-    assert e.value == -7.0 and bool((f == 5.0).all())
-    bonds(b, f)
-    assert not bool((f == 5.0).any())
+        evaluate(wrong)
+    torch.cuda.synchronize()
+    assert e.value == -7.0 and list(pr) == [-7.0] * 3 and clamped.value == -7
+    assert all(bool((v == 5.0).all()) for v in out)
+    evaluate(members)
+    torch.cuda.synchronize()
+    assert not bool((out[0] == 5.0).any()) and bool(torch.isfinite(out[0]).all())
+    if term == "dihedrals":
+        assert not bool((out[1] == 5.0).any()) and not bool((out[2] == 5.0).any())
 
 
 @pytest.mark.parametrize("T", [1, 2, 3, 4, 5, 6, 7, 8])
