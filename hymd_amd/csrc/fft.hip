@@ -206,11 +206,15 @@ struct RealSplit {
     }
 };
 
-// -i kd v for a derivative factor kd, in FP32 or (wide) in FP64
-__device__ __forceinline__ float2 mul_minus_i(float2 v, double kd, bool wide) {
-    if (wide) return make_float2((float)(kd * (double)v.y), (float)(-kd * (double)v.x));
-    const float k = (float)kd;
-    return make_float2(k * v.y, -k * v.x);
+// -i k v for a derivative factor k, zero on its Nyquist plane, in FP32 or (wide)
+// in FP64
+__device__ __forceinline__ float2 mul_minus_i(float2 v, double k, bool nyquist, bool wide) {
+    if (wide) {
+        const double kd = nyquist ? 0.0 : k;
+        return make_float2((float)(kd * (double)v.y), (float)(-kd * (double)v.x));
+    }
+    const float kd = nyquist ? 0.f : (float)k;
+    return make_float2(kd * v.y, -kd * v.x);
 }
 
 // Its inverse: Z'[m] = (X[m] + X*[nh-m]) + i conj(post[m]) (X[m] - X*[nh-m])
@@ -268,17 +272,17 @@ static YzArgs yz_args(const FftPlan &plan, const YzJob &job) {
 // the y line, so its factor commutes with the transform; both zero on their
 // Nyquist planes).
 struct YzFactor {
-    bool dy, dz, wide;
+    bool dy, dz, wide, nyquist;
     int y, my;
     double kfy, kz;
     __device__ YzFactor(const YzGrid &q, int y_, int m, int my_, int nh)
-        : dy(q.dy), dz(q.dz), wide(q.wide), y(y_), my(my_), kfy(q.kfy), kz(m == nh ? 0.0 : q.kfz * m) {}
+        : dy(q.dy), dz(q.dz), wide(q.wide), nyquist(m == nh), y(y_), my(my_), kfy(q.kfy), kz(q.kfz * m) {}
     __device__ float2 operator()(float2 v, int d) const {
         if (dy) {
             const int yy = y + d;
-            return mul_minus_i(v, 2 * yy == my ? 0.0 : kfy * (2 * yy < my ? yy : yy - my), wide);
+            return mul_minus_i(v, kfy * (2 * yy < my ? yy : yy - my), 2 * yy == my, wide);
         }
-        return dz ? mul_minus_i(v, kz, wide) : v;
+        return dz ? mul_minus_i(v, kz, nyquist, wide) : v;
     }
 };
 
@@ -446,7 +450,7 @@ __global__ void __launch_bounds__(NT, WPE) c2r_yz_plane_kernel_fixed(YzArgs a, P
         float2 w = src[y * zh + kz];
         if (q.dy) {  // row y: k_y, zero on the Nyquist row
             const int ny = 2 * y < my ? y : y - my;
-            w = mul_minus_i(w, 2 * y == my ? 0.0 : q.kfy * ny, WIDE);
+            w = mul_minus_i(w, q.kfy * ny, 2 * y == my, WIDE);
         }
         return w;
     });
@@ -458,8 +462,8 @@ __global__ void __launch_bounds__(NT, WPE) c2r_yz_plane_kernel_fixed(YzArgs a, P
         const int p = nh - m;
         float2 xm = row[m], xp = row[p];
         if (q.dz) {  // column kz: k_z, zero on the Nyquist column
-            xm = mul_minus_i(xm, 2 * m == mz ? 0.0 : q.kfz * m, WIDE);
-            xp = mul_minus_i(xp, 2 * p == mz ? 0.0 : q.kfz * p, WIDE);
+            xm = mul_minus_i(xm, q.kfz * m, 2 * m == mz, WIDE);
+            xp = mul_minus_i(xp, q.kfz * p, 2 * p == mz, WIDE);
         }
         const float2 sm = cadd(xm, cconj(xp));
         const float2 df = cmul(cconj(s.post[m]), csub(xm, cconj(xp)));
