@@ -366,8 +366,7 @@ static Workspace &workspace() {
 // Sums of the partials (nv values, 0: none) and the index check of a call
 // whose lists were built unchecked, in one synchronising read-back; a call
 // waits for the GPU once.  (Peptides of 81k beads, bonds, angles and dihedrals
-// with energies: six read-backs before, three now,
-// 358 -> 264 us.)
+// with energies: six read-backs took 348 to 363 us, three 238 to 264.)
 static int finish_terms(Workspace &w, int nblocks, int nv, double *out, int64_t n, hipStream_t s) {
     constexpr size_t bytes = sizeof(double) * (Workspace::kSums + 1);
     HYMD_TRY(w.host.reserve(bytes));

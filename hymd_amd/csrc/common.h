@@ -193,7 +193,7 @@ __device__ __forceinline__ int rank_in_bin_all(int key, int *counts) {
 // count.  Each wavefront enters the items that share its first item's bin as
 // one, so they do not queue on one slot.  Ordered wavefronts of one mesh row
 // wait on the same counter: 16.8M positions on 256^2 rows took 407 us with
-// rank_in_bin_all, 220 us here, 2.1M on 128 x 120 rows 34 and 25 us.
+// rank_in_bin_all, 249 us here, 2.1M on 128 x 120 rows 34 and 31 us.
 // Unordered items take rank_in_bin_all, which has no table to clear (351k on
 // 6480 rows: 14.7 us, 18.7 us through the table).  Every thread of the
 // workgroup must call it, once per table.

@@ -2,13 +2,16 @@
 //
 // What bounds the transforms of this path is neither flops nor HBM but the
 // passes over LDS between the stages and the index arithmetic around them, so
-// a line takes as few stages as possible (two for every length to 256 but
-// 125, 162, 200, 216, 243 and 250, three to 1024 but 625): the first stage
-// reads its elements from wherever they are (global memory, or LDS through
-// an element-wise map), the last one hands its outputs to a store functor, and
-// only the values between two stages cross LDS.  Butterfly indices are split
-// by a float reciprocal (exact below 2^22, see divq), five full-rate
-// instructions where an integer multiply-high takes three quarter-rate ones.
+// a line takes as few stages as possible.  With radices up to 10, as the line
+// and plane passes take them: two to 100 points but for 75 and 96, three to
+// 1000 but for 375, 625, 675, 750, 768, 864, 960 and 972; the x-line pass of one
+// and two types ends with a radix up to 16 and takes two to 160 points.  The
+// first stage reads its elements from wherever they are (global memory, or LDS
+// through an element-wise map), the last one hands its outputs to a store
+// functor, and only the values between two stages cross LDS.  Butterfly indices
+// are split by a float reciprocal (exact below 2^22, see divq), five
+// full-rate instructions where an integer multiply-high takes three quarter-rate
+// ones.
 //
 // Stage s of radix R after sub-transforms of size p (self-sorting Stockham):
 // butterfly i of n/R, k = i mod p, reads x[i + j n/R], multiplies by
@@ -66,8 +69,9 @@ struct LineAxis {
 };
 
 // q = b / d for 0 <= b < 2^22 and inv = 1.0f / d: (b + 0.5) / d lies at least
-// 0.5 / d from an integer, and the two roundings move it by less than
-// b / d * 2^-22 <= 0.5 / d * 2^-21 b.
+// 0.5 / d from an integer, and the two roundings, of 2^-24 each, move it by
+// less than (b + 0.5) / d * 2^-23 (1 + 2^-24), which stays below 0.5 / d while
+// b + 1 <= 2^22.
 __device__ __forceinline__ int divq(int b, float inv) { return (int)(((float)b + 0.5f) * inv); }
 
 // ---------------------------------------------------------------------------
@@ -258,14 +262,10 @@ struct Dft<16, SGN> {
 
 }  // namespace dft
 
-// Calls op(std::integral_constant<int, R>) for a radix R <= MAXR of the plans.
+// Calls op(std::integral_constant<int, R>) for a radix R <= MAXR <= 10 of the plans.
 template <int MAXR, class Op>
 __device__ __forceinline__ void with_radix(int R, Op &&op) {
-    if constexpr (MAXR > 10) {
-        if (R == 12) return op(std::integral_constant<int, 12>{});
-        if (R == 15) return op(std::integral_constant<int, 15>{});
-        if (R == 16) return op(std::integral_constant<int, 16>{});
-    }
+    static_assert(MAXR <= 10, "radices of a stage that goes through LDS");
     if constexpr (MAXR > 8) {
         if (R == 9) return op(std::integral_constant<int, 9>{});
         if (R == 10) return op(std::integral_constant<int, 10>{});

@@ -151,6 +151,7 @@ __global__ void __launch_bounds__(NT) xline_fixed_kernel(const float2 *__restric
 template <int MAXT, int NT, int T, int N, int W, bool PME>
 static int launch_fixed(const FftPlan &plan, const XlineJob &job, int blocks, hipStream_t s) {
     using G = XlineFixed<T, N, W>;
+    static_assert(T <= MAXT && W * N <= NT * (16 / MAXT), "every position of the W lines is held by a thread");
     const size_t lds = sizeof(float2) * ((size_t)N + (size_t)T * W * (N + 1));
     static bool done = false;  // the opt-in is per kernel and process
     if (!done && lds > 64 * 1024) {
