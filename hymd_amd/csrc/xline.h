@@ -133,8 +133,15 @@ __device__ __forceinline__ int fresh(int v) {
     return v;
 }
 
+// Waves per SIMD that the registers allow: four where they suffice; the 15 and
+// 16 elements of psi and of -i k_x psi of a PME thread spilled 36 to 60 bytes a
+// lane at four (150 x 144 x 160 21.0 us), and are faster at three (18.4).
+constexpr int xline_waves(int T, int R2, bool pme) {
+    return T * R2 > 16 ? 1 : (pme && R2 > 12 ? 3 : 4);
+}
+
 template <int T, int R2, bool PME, class G>
-__global__ void __launch_bounds__(G::threads, T * R2 <= 16 ? 4 : 1)
+__global__ void __launch_bounds__(G::threads, xline_waves(T, R2, PME))
     xline_kernel(const float2 *__restrict__ spec, float2 *__restrict__ out, float2 *__restrict__ phif,
                  float2 *__restrict__ phix, XlineArgs a, G geo, KGeom g, FieldK p, PmeK pk,
                  double *__restrict__ partials) {
