@@ -725,10 +725,11 @@ static int lds_opt_in(K kernel, bool &done) {
 }
 
 // Calls f(geometry, threads) with the plane geometry for `planes` planes of
-// the plan in one direction: compile-time for the planes of the cubic meshes listed, whose
-// sizes the package's workloads use (128^2 on fft_ct.h, the four types of a
-// lipid/water step: c2r 48 us against 68 for the general form), else the
-// general one.
+// the plan in one direction: compile-time for the planes of the cubic meshes
+// listed, whose sizes the package's workloads use, else the general one.  Four
+// types, c2r and r2c: 128^2 on fft_ct.h 48 us against 68 for the general form
+// (c2r), 96^2 23.9 and 11.6 against 28.5 and 14.0, 64^2 9.3 and 6.0 against 11.1
+// and 8.4, 48^2 7.2 and 4.8 against 8.8 and 6.8; whole updates 5 to 9 %.
 template <class F>
 static int with_plane(const FftPlan &plan, int64_t planes, bool inverse, F &&f) {
     const Mesh &m = plan.mesh;
