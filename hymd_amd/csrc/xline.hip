@@ -48,6 +48,21 @@ XlineShape xline_shape(const FftPlan &plan, int T, int want, bool fixed) {
             if (fits(W, kXlineLdsBytes)) sh.W = W;
     }
     sh.threads = sh.W ? threads(sh.W) : 0;
+    // One line of one or two types (which keep the pass, xline_narrow): two or
+    // four, where the middle stages need at most a quarter more threads for them
+    // than the others.  900 x 96 x 96, one type 257 us with one line, 224 with
+    // four; 900 x 256 x 256 2619 and 1574, its PME 2657 and 1632; 450 x 96 x 96, two
+    // types 210 and 186.  (810 x 96 x 96, two types: half as many more, 366 and 382.)
+    for (int W = 4; W >= 2 && T <= 2 && sh.W == 1; W >>= 1) {
+        int t = threads(W);
+        for (int s = 1; s < ax.ns - 1; ++s) {
+            const int held = std::max(1, kXlineElems / ax.st[s].R);
+            t = std::max(t, ((T * W * ax.st[s].nr + held - 1) / held + 63) / 64 * 64);
+        }
+        if (t > kXlineThreads || 4 * t > 5 * threads(W) || xline_lds(n, T, W) > 80 * 1024) continue;
+        sh.W = W;
+        sh.threads = t;
+    }
     return sh;
 }
 
