@@ -62,14 +62,16 @@ inline int xline_fixed_lines(int n, int T, int want) {
 //   plane measured (64 to 256 rows of 33 to 161 elements; the strides seem to
 //   meet on few memory channels):
 //     W = 2: T = 6, 192 x 256 x 256 2305 / 1735, 240 x 256 x 256 2668 / 2228.
-//     W = 4: T = 4, 192 x 256 x 256 1123 / 1175; T = 6, 100 x 256 x 256 908 / 938,
+//     W = 4: T = 4, 192 x 256 x 256 1123 / 1175; T = 6, 100 x 256 x 256 908 / 938;
 //       but where the types lie 2^k 129 elements apart as well T = 8, 128 x 256 x
-//       256 2000 / 1563, T = 6, 96 x 256 x 256 951 / 896.
+//       256 2000 / 1563, T = 6, 96 x 256 x 256 951 / 896, and on long lines of
+//       three types and more T = 4, 288 x 256 x 256 1945 / 1846, 320 x 256 x 256
+//       2121 / 2003, 270 x 256 x 256 1731 / 1714 (T = 2, 400 x 256 x 256 1287 / 1461).
 //     more: held spectra, W = 2, 256^3, T = 6 2488 / 1653; W = 4, 192 x 256 x 256,
 //       T = 4 874 / 825; densities, 288 x 256 x 256, T = 4 2429 / 2306.
 inline bool xline_narrow(const Mesh &m, int T, int W, bool more) {
     const bool few_channels = m.zh == 129 && m.my % 64 == 0;
-    const int least = more || (T >= 6 && m.mx % 32 == 0) ? 4 : 2;
+    const int least = more || (T >= 3 && m.mx >= 256) || (T >= 6 && m.mx % 32 == 0) ? 4 : 2;
     return (W == 1 && T >= 3) || (W == 2 && T >= 8) || (few_channels && W <= least);
 }
 
