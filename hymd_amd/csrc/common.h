@@ -360,6 +360,7 @@ int update_field_force_q_impl(hymd_pm *pm, const float *x, const float *charges,
 uint64_t pm_generation(const hymd_pm *pm);
 // the handle's current box edges
 void pm_box(const hymd_pm *pm, double box[3]);
+hipStream_t pm_stream(const hymd_pm *pm);
 // a new handle with src's mesh and box (own buffers and plans)
 int pm_clone(const hymd_pm *src, int32_t max_types, void *stream, hymd_pm **out);
 

@@ -734,6 +734,8 @@ int hymd::pm_clone(const hymd_pm *src, int32_t max_types, void *stream, hymd_pm 
     return hymd_pm_create(out, mesh, src->mesh.box, max_types, stream);
 }
 
+hipStream_t hymd::pm_stream(const hymd_pm *pm) { return pm->stream; }
+
 void hymd::pm_box(const hymd_pm *pm, double box[3]) {
     for (int d = 0; d < 3; ++d) box[d] = pm->mesh.box[d];
 }

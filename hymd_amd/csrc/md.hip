@@ -151,13 +151,26 @@ __global__ void __launch_bounds__(kBlock) reorder_store_kernel(int64_t ns, int64
     }
 }
 
+// The caller's mesh handle on a stream of the MD handle for the length of a
+// scope; its own stream again after it.  (Left on `work` the handle pointed at
+// a destroyed stream once hymd_md_destroy had run, and its own destruction
+// synchronised that.)
+struct PmOnStream {
+    hymd_pm *pm;
+    hipStream_t before;
+    PmOnStream(hymd_pm *p, hipStream_t s) : pm(p), before(pm_stream(p)) { (void)hymd_pm_set_stream(pm, s); }
+    ~PmOnStream() { (void)hymd_pm_set_stream(pm, before); }
+    PmOnStream(const PmOnStream &) = delete;
+    PmOnStream &operator=(const PmOnStream &) = delete;
+};
+
 static int reorder_singles(hymd_md *m) {
     const int64_t s0 = m->single0, ns = m->n - s0;
     if (ns <= 1) return HYMD_OK;
     hipStream_t s = m->work;
     HYMD_TRY(m->rperm.reserve(sizeof(int) * ns));
     HYMD_TRY(m->rtmp.reserve((sizeof(double) * 6 + sizeof(float) * 9 + sizeof(int32_t) + sizeof(int64_t)) * ns));
-    HYMD_TRY(hymd_pm_set_stream(m->pm, s));
+    const PmOnStream on(m->pm, s);
     HYMD_TRY(row_order(m->pm, m->x32 + 3 * s0, ns, (int *)m->rperm.ptr, s));
     char *p = (char *)m->rtmp.ptr;
     ReorderArrays t;
@@ -306,7 +319,7 @@ static int fused_inner(hymd_md *m, int pending, double *energies, double *virial
 static int enqueue_step(hymd_md *m, double *energies, int pending) {
     const double half_in = 0.5 * m->dt / m->mass;
     const double half_out = 0.5 * m->respa_inner * m->dt / m->mass;
-    HYMD_TRY(hymd_pm_set_stream(m->pm, m->work));
+    const PmOnStream on(m->pm, m->work);
     if (m->fused) {
         // fused: the step ends after the slow forces; its outer half kick is
         // applied by the next step's kernel (or by finish_pending)
@@ -420,7 +433,7 @@ static int enqueue_half(hymd_md *m, int part, double *virials, double *energies)
     const bool extra = m->charges || m->dih;
     float *f_slow = extra ? m->f_slow : m->f_field;
     const int64_t n3 = 3 * m->n;
-    HYMD_TRY(hymd_pm_set_stream(m->pm, m->work));
+    const PmOnStream on(m->pm, m->work);
     if (part == 0) {
         if (m->fused) {
             HYMD_TRY(fused_inner(m, m->pending, energies, virials, nullptr));

@@ -537,3 +537,31 @@ def test_captured_step_follows_pm_buffer_growth_and_box(hip):
     assert float(a.x.max()) < float(new_box[0]) and float(a.x.max()) > float(s.box[0]) * 0.99
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("reorder_every", [0, 1])
+def test_mesh_handle_keeps_its_stream(hip, reorder_every):
+    """The MD handle runs the caller's mesh handle on a stream of its own during
+    a step and gives it back its own stream: a transform called on the bare
+    handle (without setting a stream first) after the MD handle, and with it that
+    stream, is gone runs on the stream the mesh handle had before."""
+    from hymd_amd import _lib, synth
+    from hymd_amd._lib import call, dptr
+    from hymd_amd.md import RespaMD
+    s = synth.lipid_water(n_chains=300, n_water=2000, box=6.0, mesh=16, seed=7)
+    md = RespaMD(s, reorder_every=reorder_every)
+    own = torch.cuda.Stream()
+    call("hymd_pm_set_stream", md.pm._h, own.cuda_stream)
+    md.run(2)
+    md.run(1, energies=True)
+    torch.cuda.synchronize()
+    _lib.lib().hymd_md_destroy(md._native)
+    md._native = None
+    grid = torch.rand(16, 16, 16, device="cuda")
+    out = torch.zeros(16, 16, 9, dtype=torch.complex64, device="cuda")
+    torch.cuda.synchronize()
+    call("hymd_fft_r2c", md.pm._h, dptr(grid, torch.float32), dptr(out, torch.complex64), 1)
+    own.synchronize()
+    want = torch.fft.rfftn(grid.double())
+    assert float((out - want).abs().max()) < 1e-4 * float(want.abs().max())
+    md.close()
