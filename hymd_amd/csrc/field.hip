@@ -1145,9 +1145,10 @@ static int kspace_pass(hymd_pm *pm, const FieldK &p, bool transformed, float2 *p
     job.g = kgeom(pm);
     job.p = p;
     job.partials = partials;
-    const bool more = phif || phix || transformed;
-    const XlineShape sh = xline_shape(pm->fft, T, pm->xline_w, !more);
-    const bool narrow = sh.W != pm->xline_w && xline_narrow(m, T, sh.W, more);  // a width asked for is taken
+    const bool densities = phif || phix;
+    const XlineShape sh = xline_shape(pm->fft, T, pm->xline_w, !densities && !transformed);
+    // a width asked for is taken
+    const bool narrow = sh.W != pm->xline_w && xline_narrow(m, T, sh.W, densities, transformed);
     if (sh.W > 0 && fused && !narrow) return xline_pass(pm->fft, sh, job, nblocks, s);
     if (!transformed) HYMD_TRY(fft_forward_x(pm->fft, (float2 *)pm->spec.ptr, T, s));
     if (phix && !phif) phif = phix;

@@ -50,13 +50,16 @@ inline int xline_fixed_lines(int n, int T, int want) {
 }
 
 // Whether W lines per workgroup (runs of 8 W bytes) are too few for the pass,
-// so that the separate passes (16 lines each) are the faster ones.  more: the
-// job also writes spectra and densities, or starts from held spectra; else it
-// makes the force grids only.  The whole call with the pass / separate, us:
+// so that the separate passes (16 lines each) are the faster ones.  densities:
+// the job writes spectra or densities too; transformed: it starts from held
+// spectra; else it makes the force grids only.  The whole call with the pass /
+// separate, us:
 //   W = 1: 216^3, T = 8 2316 / 2093; 240^3, T = 8 2978 / 2643; up to two types
 //     keep it: 900 x 96 x 96, T = 1 251 / 263.
-//   W = 2: T = 8, 144^3 639 / 580, 160^3 687 / 645, 200^3 1539 / 1560; fewer
-//     types keep it: T = 6, 216^3 1460 / 1608, 240^3 1819 / 2002.
+//   W = 2: T = 8, 144^3 639 / 580, 160^3 687 / 645, 200^3 1539 / 1560; with
+//     densities it goes either way (144^3 828 / 771, 160 x 180 x 216 1595 / 1620,
+//     192^3 1603 / 1687) and they keep it, as fewer types do: T = 6, 216^3 1460 /
+//     1608, 240^3 1819 / 2002.
 //   Rows of 129 elements in multiples of 64, where the x stride is 2^k 129
 //   elements and the pass moves 0.8 to 1.6 TB/s against 1.7 to 2.0 on every other
 //   plane measured (64 to 256 rows of 33 to 161 elements; the strides seem to
@@ -67,12 +70,13 @@ inline int xline_fixed_lines(int n, int T, int want) {
 //       256 2000 / 1563, T = 6, 96 x 256 x 256 951 / 896, and on long lines of
 //       three types and more T = 4, 288 x 256 x 256 1945 / 1846, 320 x 256 x 256
 //       2121 / 2003, 270 x 256 x 256 1731 / 1714 (T = 2, 400 x 256 x 256 1287 / 1461).
-//     more: held spectra, W = 2, 256^3, T = 6 2488 / 1653; W = 4, 192 x 256 x 256,
-//       T = 4 874 / 825; densities, 288 x 256 x 256, T = 4 2429 / 2306.
-inline bool xline_narrow(const Mesh &m, int T, int W, bool more) {
+//     Held spectra, W = 2, 256^3, T = 6 2488 / 1653; W = 4, 192 x 256 x 256,
+//       T = 4 874 / 825; with densities, 288 x 256 x 256, T = 4 2429 / 2306.
+inline bool xline_narrow(const Mesh &m, int T, int W, bool densities, bool transformed) {
+    const bool more = densities || transformed;
     const bool few_channels = m.zh == 129 && m.my % 64 == 0;
     const int least = more || (T >= 3 && m.mx >= 256) || (T >= 6 && m.mx % 32 == 0) ? 4 : 2;
-    return (W == 1 && T >= 3) || (W == 2 && T >= 8) || (few_channels && W <= least);
+    return (W == 1 && T >= 3) || (W == 2 && T >= 8 && !densities) || (few_channels && W <= least);
 }
 
 struct XlineJob {
